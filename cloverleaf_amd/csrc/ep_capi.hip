@@ -1013,18 +1013,69 @@ int ep_set_table(ep_ctx* c, const float* rows) {
   return EP_OK;
 }
 
+// Copies a rows x D FP32 array that the device holds in another layout: stage(first, count,
+// dst) fills dst with rows [first, first + count) on the context's stream, at most 64 MiB of
+// them at a time (halved while that cannot be allocated), each chunk copied out in one piece.
+// *staged is false when no device memory was left to stage in (nothing was copied then).
+extern "C++" template <typename Stage>
+static int copy_staged(ep_ctx* c, float* out, uint64_t rows, uint32_t D, bool* staged, Stage stage) {
+  const uint64_t row_bytes = (uint64_t)D * sizeof(float);
+  uint64_t chunk = std::min<uint64_t>(rows, std::max<uint64_t>(((uint64_t)64 << 20) / row_bytes, 1));
+  float* buf = nullptr;
+  *staged = false;
+  while (hipMalloc((void**)&buf, chunk * row_bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    if (chunk == 1) return EP_OK;
+    chunk = (chunk + 1) / 2;
+  }
+  *staged = true;
+  hipError_t e = hipSuccess;
+  for (uint64_t r = 0; r < rows && e == hipSuccess; r += chunk) {
+    const uint64_t n = std::min(chunk, rows - r);
+    e = stage(r, n, buf);
+    if (e == hipSuccess) e = hipMemcpyAsync(out + r * D, buf, n * row_bytes, hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  }
+  (void)hipFree(buf);
+  if (e != hipSuccess) return fail(EP_EHIP, std::string("staged copy: ") + hipGetErrorString(e));
+  return EP_OK;
+}
+
+// One D-wide part of the optimizer records (master, m or v) to out[n_vocab * D]: packed on the
+// device first (a pitched copy moves row by row), pitched only when there is no memory left.
+static int copy_record_part(ep_ctx* c, const float* part, uint32_t D, uint32_t ostride, float* out) {
+  bool staged = false;
+  EP_TRY(copy_staged(c, out, c->n_vocab, D, &staged, [&](uint64_t r, uint64_t n, float* dst) {
+    return ep::launch_pack_rows(part + r * ostride, dst, n, D, ostride, c->stream);
+  }));
+  if (!staged)
+    EP_HIP(hipMemcpy2D(out, D * sizeof(float), part, ostride * sizeof(float), D * sizeof(float), c->n_vocab,
+                       hipMemcpyDeviceToHost));
+  return EP_OK;
+}
+
+// MI355X host: 8.4M values take 3.3 ms either way, 25.6M 9.9 ms against 18.6 on the host, 4.2M
+// 1.1 ms against 0.84.
+constexpr size_t kWidenOnDevice = (size_t)1 << 23;
+
 int ep_get_table(ep_ctx* c, float* rows) {
   if (!c || !rows) return fail(EP_EINVAL, "NULL argument");
   if (!c->table_ready) return fail(EP_ESTATE, "no table");
   EP_HIP(hipSetDevice(c->device));
-  const size_t n = (size_t)c->n_vocab * row_width(c->cfg);
   const uint32_t D = row_width(c->cfg);
   EP_HIP(hipStreamSynchronize(c->stream));
-  if (c->cfg.precision == EP_PREC_BF16_MASTER) {
-    EP_HIP(hipMemcpy2D(rows, D * sizeof(float), c->d_ostate, 3 * D * sizeof(float), D * sizeof(float), c->n_vocab,
-                       hipMemcpyDeviceToHost));
-  } else if (c->cfg.precision == EP_PREC_BF16) {
-    // the bf16 table is the parameter: widen it (exact)
+  if (c->cfg.precision == EP_PREC_BF16_MASTER) return copy_record_part(c, c->d_ostate, D, 3 * D, rows);
+  const size_t n = (size_t)c->n_vocab * D;
+  if (c->cfg.precision == EP_PREC_BF16) {
+    // the bf16 table is the parameter, widened (exact) on the device from kWidenOnDevice
+    // values up; smaller tables, where the staging buffer's allocation costs more than the
+    // widening, and tables with no memory left to stage in, here
+    bool staged = false;
+    if (n >= kWidenOnDevice)
+      EP_TRY(copy_staged(c, rows, c->n_vocab, D, &staged, [&](uint64_t r, uint64_t k, float* dst) {
+        return ep::launch_widen_bf16((const uint16_t*)c->d_table + r * D, dst, k * D, c->stream);
+      }));
+    if (staged) return EP_OK;
     std::vector<uint16_t> h(n);
     EP_HIP(hipMemcpy(h.data(), c->d_table, n * sizeof(uint16_t), hipMemcpyDeviceToHost));
     for (size_t i = 0; i < n; ++i) {
@@ -1052,13 +1103,10 @@ int ep_get_adam(ep_ctx* c, float* m, float* v) {
   EP_HIP(hipSetDevice(c->device));
   const uint32_t D = row_width(c->cfg);
   const bool ms = c->cfg.precision == EP_PREC_BF16_MASTER;
-  const size_t ostride = (ms ? 3 : 2) * (size_t)D;
+  const uint32_t ostride = (ms ? 3u : 2u) * D;
   EP_HIP(hipStreamSynchronize(c->stream));
-  EP_HIP(hipMemcpy2D(m, D * sizeof(float), c->d_ostate + (ms ? D : 0), ostride * sizeof(float), D * sizeof(float),
-                     c->n_vocab, hipMemcpyDeviceToHost));
-  EP_HIP(hipMemcpy2D(v, D * sizeof(float), c->d_ostate + (ms ? 2 * D : D), ostride * sizeof(float),
-                     D * sizeof(float), c->n_vocab, hipMemcpyDeviceToHost));
-  return EP_OK;
+  EP_TRY(copy_record_part(c, c->d_ostate + (ms ? D : 0u), D, ostride, m));
+  return copy_record_part(c, c->d_ostate + (ms ? 2u * D : D), D, ostride, v);
 }
 
 int ep_set_split(ep_ctx* c, const uint32_t* train, uint64_t n_train, const uint32_t* valid, uint64_t n_valid) {
