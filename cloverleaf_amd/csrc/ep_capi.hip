@@ -1459,6 +1459,18 @@ int ep_step_explicit_noalloc(ep_ctx* c, const uint32_t* anchors, uint32_t n, con
   return EP_OK;
 }
 
+// Rows updated so far by the short-row kernel, and by every update path.
+static uint64_t short_rows_updated(const ep::StepState& st) {
+  uint64_t n = 0;
+  for (unsigned long long x : st.upd_short) n += x;
+  return n;
+}
+static uint64_t rows_updated(const ep::StepState& st) {
+  uint64_t n = st.stat_unique + short_rows_updated(st);
+  for (unsigned long long x : st.upd_long) n += x;
+  return n;
+}
+
 int ep_bench_steps(ep_ctx* c, uint32_t warmup, uint32_t steps, int instrument, ep_bench_result* out) {
   if (!c || !out || steps == 0) return fail(EP_EINVAL, "bad argument");
   std::memset(out, 0, sizeof(*out));
@@ -1520,7 +1532,7 @@ int ep_bench_steps(ep_ctx* c, uint32_t warmup, uint32_t steps, int instrument, e
   out->examples = h1.stat_examples - h0.stat_examples;
   out->rows = h1.stat_rows - h0.stat_rows;
   out->nodes = h1.stat_nodes - h0.stat_nodes;
-  out->unique_rows = h1.stat_unique - h0.stat_unique;
+  out->unique_rows = rows_updated(h1) - rows_updated(h0);
   out->att_items_sq = h1.stat_att_n2 - h0.stat_att_n2;
   out->att_items = h1.stat_att_n - h0.stat_att_n;
   out->seg_vpl = c->seg_vpl;
@@ -1550,7 +1562,7 @@ int ep_bench_steps(ep_ctx* c, uint32_t warmup, uint32_t steps, int instrument, e
     for (int k = 0; k < 8; ++k) out->ms_phase[k] = ph[k] / steps;
     out->ms_forward_avg = out->ms_phase[1];
     out->ms_scatter_avg = out->ms_phase[3] + out->ms_phase[4] + out->ms_phase[5] + out->ms_phase[6] + out->ms_phase[7];
-    out->short_rows = g1.stat_short - g0.stat_short;
+    out->short_rows = short_rows_updated(g1) - short_rows_updated(g0);
     out->last_long_rows = g1.n_long;
     out->last_pieces = g1.n_pieces;
     out->forward_launches = steps;

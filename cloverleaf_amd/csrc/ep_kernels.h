@@ -23,9 +23,8 @@ struct StepState {
   uint64_t next_step;      // LR-schedule step counter (1-based, like the reference's AtomicUsize)
   uint64_t stat_rows;      // cumulative feature-row reads (sum of R_e)
   uint64_t stat_nodes;     // cumulative node-id reads (sampled neighbours + negatives)
-  uint64_t stat_unique;    // cumulative unique rows updated
+  uint64_t stat_unique;    // cumulative unique rows updated by the atomic path
   uint64_t stat_examples;  // cumulative anchors processed
-  uint64_t stat_short;     // cumulative rows updated by the short-row kernel
   uint64_t stat_att_n2;    // attention: cumulative sum over blocks of items^2
   uint64_t stat_att_n;     // attention: cumulative sum over blocks of items
   uint32_t pass;           // 1-based pass
@@ -47,6 +46,9 @@ struct StepState {
   uint32_t n_real;         // non-sentinel keys (the sorted key count)
   uint32_t reg_next;       // next plan region for k_seg_update (cleared by k_seg_plan)
   uint32_t dtot[4][2048];  // radix-sort digit totals, one row per sort pass (<= 11-bit digits)
+  // cumulative rows updated, one slot per block of the row kernels: by the short-row kernel,
+  // and by the medium- and long-row kernels (stat_unique: by the atomic path)
+  unsigned long long upd_short[2048], upd_long[2048];
 };
 
 // Static description of the step (fixed for the life of a captured graph).

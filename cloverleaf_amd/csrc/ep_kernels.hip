@@ -13,6 +13,9 @@
 #include "ep_kernels.h"
 #include "ep_loss.h"
 
+#include <algorithm>
+#include <atomic>
+
 namespace ep {
 
 static constexpr int NW = kBlockWaves;   // waves per 256-thread block
@@ -1843,6 +1846,10 @@ __device__ inline void adam_math(float& th, float& m, float& v, float g, float l
   th -= lr * (m * ibc1) * __builtin_amdgcn_rcpf(den);
 }
 
+// k_seg_update's units (see there): a region's rows go to at most kUpdSplitMax units, about
+// kUpdUnitsPerWave per wave of the grid.
+static constexpr uint32_t kUpdSplitMax = 16, kUpdUnitsPerWave = 2;
+
 // Per-step scalars of the update, read once per kernel (before any store, so the
 // compiler keeps them in registers instead of reloading them after each store).
 struct StepScalars {
@@ -2224,6 +2231,22 @@ __global__ __launch_bounds__(256) void k_seg_plan(StepConfig c, StepState* st, c
   }
 }
 
+// Adds the block's rows updated (x summed over its threads) to its own counter slot: blocks
+// of one stream's kernels follow each other, so no atomics.  One 64-bit atomic per wave on
+// one address serialised thousands of waves at the end of every row kernel.
+__device__ inline void count_rows(unsigned long long* slots, uint32_t x) {
+  __shared__ uint32_t s_cnt[NW];
+  x = wave_sum_u32(x);
+  if ((threadIdx.x & 63u) == 0u) s_cnt[threadIdx.x >> 6] = x;
+  __syncthreads();
+  if (threadIdx.x == 0u) {
+    uint32_t t = 0u;
+#pragma unroll
+    for (int q = 0; q < NW; ++q) t += s_cnt[q];
+    if (t) slots[blockIdx.x] += t;
+  }
+}
+
 // Short rows: lane groups of L = D/VPL lanes (VPL values per lane as VPL/4 float4
 // columns strided by L), G = 64/L rows per wave, U adjoint rows in flight per group.
 // Every (VPL, U) adds each run's rows in entry order: identical bits, so the tuner picks
@@ -2256,12 +2279,22 @@ __global__ __launch_bounds__(256) void k_seg_update(StepConfig c, StepState* st,
   __syncthreads();
   const bool noisy = c.noise > 1e-9f;
   uint32_t done = 0;
-  // wave gw takes region gw, then (only when there are more regions than waves) regions
-  // waves, waves + 1, ... from the queue: small steps make no atomics at all
+  // More regions than waves: wave gw takes region gw, then regions waves, waves + 1, ... from
+  // the queue.  Otherwise a region's rows are dealt to `split` units (unit u takes the row
+  // groups sub, sub + split, ... of region u % nreg, sub = u / nreg) and wave gw takes units
+  // gw, gw + waves, ...: no atomics, and no wave holds the up to 64 rows that start in one
+  // chunk of cold keys while others hold none.
   const uint32_t nwv = gridDim.x * NW;
-  uint32_t reg = blockIdx.x * NW + (uint32_t)(tid >> 6);
-  for (;;) {
-    if (reg >= nreg) break;
+  const bool queued = nreg > nwv;
+  uint32_t split = 1u;
+  if (!queued)
+    while (split < kUpdSplitMax && nreg * split < kUpdUnitsPerWave * nwv) split *= 2u;
+  const uint32_t units = nreg * split;
+  const uint32_t stride = (uint32_t)G * split;  // rows between two of a lane group's
+  for (uint32_t unit = blockIdx.x * NW + (uint32_t)(tid >> 6);;) {
+    if (unit >= units) break;
+    const uint32_t reg = queued ? unit : unit % nreg;
+    const uint32_t first = queued ? 0u : unit / nreg * (uint32_t)G;  // the unit's first row group
     const uint32_t nrec = c.scount[reg];
     const uint4* recs = c.srec + (size_t)reg * cpr * 64u;
     // Software pipeline over the region's rows: iteration k issues, back to back, the row's
@@ -2284,11 +2317,11 @@ __global__ __launch_bounds__(256) void k_seg_update(StepConfig c, StepState* st,
         out[i] = Ss[r.x + (e < (r.w & 63u) ? e : 0u)];
       }
     };
-    uint4 rec_next = load_rec((uint32_t)grp);
+    uint4 rec_next = load_rec(first + (uint32_t)grp);
     uint32_t sl_next[NS];
     load_slots(rec_next, sl_next);
-    uint4 rec_after = load_rec((uint32_t)(G + grp));
-    for (uint32_t j0 = 0; j0 < nrec; j0 += (uint32_t)G) {
+    uint4 rec_after = load_rec(first + stride + (uint32_t)grp);
+    for (uint32_t j0 = first; j0 < nrec; j0 += stride) {
       const uint32_t j = j0 + (uint32_t)grp;
       const bool has = gact && j < nrec;
       uint4 rec = rec_next;
@@ -2323,7 +2356,7 @@ __global__ __launch_bounds__(256) void k_seg_update(StepConfig c, StepState* st,
       }
       rec_next = rec_after;
       load_slots(rec_next, sl_next);
-      rec_after = load_rec(j0 + (uint32_t)(2 * G) + (uint32_t)grp);
+      rec_after = load_rec(j0 + 2u * stride + (uint32_t)grp);
       const uint32_t nruns = has ? (uint32_t)__popc(rmask) : 0u;
       uint32_t maxruns = nruns;
       if constexpr (G > 1) {
@@ -2462,16 +2495,15 @@ __global__ __launch_bounds__(256) void k_seg_update(StepConfig c, StepState* st,
         }
       }
     }
-    if (nreg <= nwv) break;
+    if (!queued) {
+      unit += nwv;
+      continue;
+    }
     uint32_t nx = 0u;
     if (lane == 0) nx = atomicAdd(&st->reg_next, 1u);
-    reg = nwv + (uint32_t)__shfl((int)nx, 0, EP_WAVE);
+    unit = nwv + (uint32_t)__shfl((int)nx, 0, EP_WAVE);
   }
-  done = wave_sum_u32(done);
-  if (lane == 0 && done) {
-    atomicAdd((unsigned long long*)&st->stat_unique, (unsigned long long)done);
-    atomicAdd((unsigned long long*)&st->stat_short, (unsigned long long)done);
-  }
+  count_rows(st->upd_short, done);
 }
 
 // Loads row f's optimizer operands (whole-wave slice layout).
@@ -2658,7 +2690,7 @@ __global__ __launch_bounds__(256) void k_pieces(StepConfig c, StepState* st, con
       }
     }
   }
-  if (lane == 0 && done) atomicAdd((unsigned long long*)&st->stat_unique, (unsigned long long)done);
+  count_rows(st->upd_long, lane == 0 ? done : 0u);
 }
 
 // One wave per long row: loads theta/m/v once, adds the pieces of each run in order and
@@ -2732,7 +2764,7 @@ __global__ __launch_bounds__(256) void k_long_combine(StepConfig c, StepState* s
       ++done;
     }
   }
-  if (lane == 0 && done) atomicAdd((unsigned long long*)&st->stat_unique, (unsigned long long)done);
+  count_rows(st->upd_long, lane == 0 ? done : 0u);
 }
 
 // ------------------------------------------------------------------------------------
@@ -3125,14 +3157,23 @@ static void radix_plan(int bits, int* passes, int* rb) {
   *rb = (bits + *passes - 1) / *passes;
 }
 
-// Blocks of 256 threads of kernel k resident on the current device at once, at most cap.
-template <typename Kernel>
-static int resident_blocks(Kernel k, int cap) {
+// Blocks of 256 threads of kernel K resident on the current device at once, at most cap.
+// The three runtime queries cost more than a launch, so the answer (a property of the built
+// kernel and the device model) is kept per kernel and device.
+template <auto K>
+static int resident_blocks(int cap) {
+  constexpr int kDevices = 64;
+  static std::atomic<int> known[kDevices];  // 0: not asked yet
   int dev = 0, ncu = 0, per = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return cap;
-  if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0) return cap;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k, 256, 0) != hipSuccess || per <= 0) return cap;
-  return per * ncu < cap ? per * ncu : cap;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kDevices) return cap;
+  int n = known[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0) return cap;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, K, 256, 0) != hipSuccess || per <= 0) return cap;
+    n = per * ncu;
+    known[dev].store(n, std::memory_order_relaxed);
+  }
+  return n < cap ? n : cap;
 }
 
 template <int RB>
@@ -3140,7 +3181,7 @@ static void launch_sort_rb(const StepConfig& c, StepState* st, hipStream_t s, in
   // whole rounds of resident scatter blocks (at 9-bit digits its tile and counters take
   // 44 KB of LDS, three blocks per CU): a last, partial round would leave part of the
   // device idle; the three kernels of a pass share the block partition
-  const int res = resident_blocks(k_rs_scatter<RB>, c.sort_grid);
+  const int res = resident_blocks<k_rs_scatter<RB>>(c.sort_grid);
   const int G = res < c.sort_grid ? (c.sort_grid / res) * res : c.sort_grid;
   for (int p = 0; p < passes; ++p) {
     const int shift = p * RB;
@@ -3230,29 +3271,38 @@ static void launch_seg_update_variant(const StepConfig& c, StepState* st, int bu
 
 
 template <int D, bool H>
-static void launch_row_kernels(const StepConfig& c, StepState* st, int buf, hipStream_t s, int grid, hipEvent_t* ev) {
-  launch_seg_update_variant<D, H>(c, st, buf, s, grid);
+static void launch_row_kernels(const StepConfig& c, StepState* st, int buf, hipStream_t s, hipEvent_t* ev) {
+  // grids that the step's largest key count can fill: blocks for `per` waves per 64-key chunk
+  const uint64_t chunks = ((uint64_t)c.key_cap + 63u) / 64u;
+  auto wave_grid = [&](uint64_t per) { return (int)std::min<uint64_t>(c.unique_grid, (chunks * per + NW - 1u) / NW); };
+  launch_seg_update_variant<D, H>(c, st, buf, s, wave_grid(kUpdSplitMax));
   if (ev) (void)hipEventRecord(ev[1], s);
   // k_pieces sweeps the pieces batch by batch: one round of resident blocks keeps every
   // wave on the same batch
-  const int pgrid = resident_blocks(k_pieces<D, H>, grid);
+  const int pgrid = resident_blocks<k_pieces<D, H>>(wave_grid(2));
   hipLaunchKernelGGL((k_pieces<D, H>), dim3(pgrid), dim3(256), 0, s, c, st, c.keys[buf], c.slots[buf]);
   if (ev) (void)hipEventRecord(ev[2], s);
   // hot rows dealt to one round of resident blocks: no late blocks holding the last rows
-  const int lgrid = resident_blocks(k_long_combine<D, H>, grid);
+  const int lgrid = resident_blocks<k_long_combine<D, H>>(wave_grid(1));
   hipLaunchKernelGGL((k_long_combine<D, H>), dim3(lgrid), dim3(256), 0, s, c, st, c.keys[buf], c.slots[buf]);
   if (ev) (void)hipEventRecord(ev[3], s);
 }
 
-hipError_t launch_scatter_sorted(const StepConfig& c, StepState* st, int buf, hipStream_t s, hipEvent_t* ev) {
-  const int grid = c.unique_grid;
+hipError_t launch_scatter_sorted(const StepConfig& c0, StepState* st, int buf, hipStream_t s, hipEvent_t* ev) {
+  // The plan's grid and regions: unique_grid blocks and n_regions regions (what the records
+  // are sized for), cut to a wave and a region per chunk when the step's largest key count
+  // has fewer chunks than that.
+  StepConfig c = c0;
+  int grid = c.unique_grid;
+  while (grid > 1 && (uint64_t)(grid / 2) * NW * 64u >= c.key_cap) grid /= 2;
+  if (grid < c.unique_grid) c.n_regions = (uint32_t)grid * NW;
   hipLaunchKernelGGL(k_seg_plan, dim3(grid), dim3(256), 0, s, c, st, c.keys[buf], c.slots[buf]);
   if (ev) (void)hipEventRecord(ev[0], s);
   if (c.adjh) {
     // FP16 adjoint rows: the mean model's widths
-    EP_DISPATCH(c.dims, { (launch_row_kernels<D, true>)(c, st, buf, s, grid, ev); });
+    EP_DISPATCH(c.dims, { (launch_row_kernels<D, true>)(c, st, buf, s, ev); });
   } else {
-    EP_ROW_DISPATCH(c.dims, { (launch_row_kernels<D, false>)(c, st, buf, s, grid, ev); });
+    EP_ROW_DISPATCH(c.dims, { (launch_row_kernels<D, false>)(c, st, buf, s, ev); });
   }
   return hipGetLastError();
 }
