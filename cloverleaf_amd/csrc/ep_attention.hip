@@ -487,6 +487,7 @@ __device__ inline void row_softmax_stats(f32x16 (&T)[2], int NT, uint32_t n, int
 __global__ __launch_bounds__(256) void k_att_map(StepConfig c, StepState* st) {
   const uint32_t lane = lane_id();
   const uint32_t b = blockIdx.x * NW + (threadIdx.x >> 6);
+  if (blockIdx.x == 0u && threadIdx.x == 0u) commit_step(st);
   if (b >= c.batch || b >= st->batch_n) return;
   const uint32_t cnt = c.nbr_cnt[b];
   if (cnt == 0u) return;

@@ -353,10 +353,27 @@ int place_step_buffers(ep_ctx* c, uint32_t batch, ep::StepConfig& b, Place&& pla
   b.fuse_emit = att ? 0 : 1;
   {
     const uint64_t words = (uint64_t)(NC + ep::kBlockWaves) * D;
+    uint64_t fwd = (words + K + 1 + NC + 1) & ~(uint64_t)1;  // even: 64-bit entries follow
     uint32_t fh = 1;
     while ((uint64_t)fh * 2 <= words) fh *= 2;
+    // a hash (and an entry byte per occurrence) for the largest example there can be, where
+    // the LDS of it costs no resident blocks: up to 16 KB in all, or what the step's blocks
+    // leave each other on 256 CUs of 160 KB.  k_emit is then never launched.
+    const uint64_t rmax = example_rows_max(c);
+    uint64_t want = fh;
+    while (want / 8 * 5 < rmax) want *= 2;
+    const uint64_t fwd_want = std::max<uint64_t>(fwd, (want + (rmax + 3) / 4 + 1) & ~(uint64_t)1);
+    const uint64_t rest = 24ull * ent_cap + 4ull * (b.ids_cap + 1024);  // entries, selections, ids, padding
+    const uint64_t room = std::max<uint64_t>(16384, std::min<uint64_t>(61440, 163840 / ((batch + 255) / 256)));
+    if (cfg.grad_mode == EP_GRAD_FIRST_LEAF && want > fh && fwd_want * 4 + rest <= room) {
+      fh = (uint32_t)want;
+      fwd = fwd_want;
+    }
+    b.fwd_words = (uint32_t)fwd;
     b.fuse_hash = fh;
     b.fuse_max = fh / 8 * 5;
+    const uint64_t entries = 1ull + neighbour_cap(c) + K;
+    b.fuse_all = !att && entries <= ent_cap && rmax <= b.ids_cap && (cfg.grad_mode != EP_GRAD_FIRST_LEAF || rmax <= b.fuse_max);
   }
   b.unique_grid = unique_grid;
   *keycap_out = keycap;
@@ -538,9 +555,7 @@ int launch_training_step(ep_ctx* c, const ep::StepConfig& sc0, bool update, floa
   pick_variant(c, sc);
   auto mark = [&](int i) -> hipError_t { return ev ? hipEventRecord(ev[i], s) : hipSuccess; };
   EP_HIP(mark(0));
-  if (lr_override >= 0.f) EP_HIP(ep::launch_step_begin_lr(sc, c->d_state, lr_override, s));
-  else EP_HIP(ep::launch_step_begin(sc, c->d_state, s));
-  EP_HIP(ep::launch_sample(sc, c->d_state, s));
+  EP_HIP(ep::launch_sample(sc, c->d_state, lr_override, s));
   EP_HIP(ep::launch_scan(sc, c->d_state, s));
   EP_HIP(mark(1));
   if (sc.model == 1) {
@@ -1177,8 +1192,7 @@ int ep_learn(ep_ctx* c, ep_progress_fn progress, void* user) {
     if (!c->valid.empty()) {
       EP_TRY(set_pass(c, c->d_vstate, 0, nullptr));
       for (uint32_t s = 0; s < vc.steps_per_pass; ++s) {
-        EP_HIP(ep::launch_step_begin_lr(vc, c->d_vstate, 0.f, c->stream));
-        EP_HIP(ep::launch_sample(vc, c->d_vstate, c->stream));
+        EP_HIP(ep::launch_sample(vc, c->d_vstate, 0.f, c->stream));
         if (vc.model == 1) {
           EP_HIP(ep::launch_scan(vc, c->d_vstate, c->stream));
           EP_HIP(ep::launch_att_forward(vc, c->d_vstate, c->stream));
@@ -1228,8 +1242,7 @@ int ep_sample_batch(ep_ctx* c, const uint32_t* anchors, uint32_t n, uint32_t pas
   sc.rbatch = n;
   EP_HIP(hipMemcpy(c->d_explicit, anchors, n * sizeof(uint32_t), hipMemcpyHostToDevice));
   EP_TRY(set_pass(c, c->d_vstate, pass, nullptr));
-  EP_HIP(ep::launch_step_begin_lr(sc, c->d_vstate, 0.f, c->stream));
-  EP_HIP(ep::launch_sample(sc, c->d_vstate, c->stream));
+  EP_HIP(ep::launch_sample(sc, c->d_vstate, 0.f, c->stream));
   EP_HIP(hipStreamSynchronize(c->stream));
   EP_HIP(hipMemcpy(nbr_cnt, sc.nbr_cnt, n * sizeof(uint32_t), hipMemcpyDeviceToHost));
   if (sc.pnbrs) {

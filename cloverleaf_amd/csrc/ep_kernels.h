@@ -16,7 +16,7 @@ constexpr int kBlockWaves = 4;
 constexpr uint32_t kSlotBatchShift = 29;
 constexpr uint32_t kSlotMask = (1u << kSlotBatchShift) - 1u;
 
-// Device-resident per-step state.  Written by k_step_begin / k_scan / the scatter
+// Device-resident per-step state.  Written by k_sample / k_scan / k_forward / the scatter
 // kernels; read by every kernel of the step, so one captured step graph can be
 // replayed for every batch of a pass.
 struct StepState {
@@ -157,10 +157,12 @@ struct StepConfig {
   uint32_t ent_cap;        // forward LDS stage: max entries (nodes) per example, <= 256
   uint32_t ids_cap;        // forward LDS stage: max feature occurrences per example
   int fuse_emit;           // k_forward emits the keys of LDS-staged examples
-  uint32_t fuse_hash;      // entries of k_forward's first-leaf hash (power of two that fits the
-                           // construction region of its LDS)
+  uint32_t fwd_words;      // 32-bit words of the forward's LDS before its id stage: constructions,
+                           // partial sums, distances, counts, then reused by the emission's hash
+  uint32_t fuse_hash;      // entries of k_forward's first-leaf hash (power of two, in fwd_words)
   uint32_t fuse_max;       // first_leaf: k_forward emits examples of at most this many
                            // occurrences (5/8 of fuse_hash), k_emit the larger ones
+  int fuse_all;            // no example can be too large for k_forward's emission: no k_emit
   // keys
   uint32_t* keys[2];
   uint32_t* slots[2];
@@ -244,11 +246,17 @@ __device__ inline const uint32_t* nbr_list(const StepConfig& c, uint32_t b, uint
 }
 
 
+// Moves the cursors past the step (the kernel after k_sample and k_scan, one thread: k_sample
+// reads them in every block).
+__device__ inline void commit_step(StepState* st) {
+  st->step_in_pass += 1u;
+  st->next_step = st->step0 + st->n_batches;
+}
+
 // Launchers (all asynchronous on `stream`).
-hipError_t launch_step_begin(const StepConfig& c, StepState* st, hipStream_t s);
-// Same, with a fixed learning rate instead of the schedule (explicit test steps).
-hipError_t launch_step_begin_lr(const StepConfig& c, StepState* st, float lr, hipStream_t s);
-hipError_t launch_sample(const StepConfig& c, StepState* st, hipStream_t s);
+// Begins a step (lr >= 0: that learning rate instead of the schedule's, explicit steps) and
+// samples its examples; launch_forward / launch_att_forward then moves the cursors on.
+hipError_t launch_sample(const StepConfig& c, StepState* st, float lr, hipStream_t s);
 hipError_t launch_scan(const StepConfig& c, StepState* st, hipStream_t s);
 hipError_t launch_forward(const StepConfig& c, StepState* st, hipStream_t s);
 hipError_t launch_emit(const StepConfig& c, StepState* st, hipStream_t s);

@@ -1,8 +1,9 @@
 // HIP kernels for one Embedding Propagation training step on gfx950 (MI355X).
 //
-// Step = k_step_begin -> k_sample -> k_scan -> k_forward -> k_emit ->
-//        {radix sort -> k_seg_adam -> k_pieces -> k_long_combine}
+// Step = k_sample -> k_scan -> k_forward -> k_emit ->
+//        {radix sort -> k_seg_plan -> k_seg_update -> k_pieces -> k_long_combine}
 //     or {k_atomic_scatter -> k_adam_touched}
+// (k_scan and k_emit only where k_forward cannot do their work itself)
 //
 // Every kernel reads the per-step values (batch offset, batch size, learning rate,
 // key count) from the device-resident StepState, so the whole step can be captured
@@ -230,39 +231,45 @@ __device__ inline float scheduled_lr(const StepConfig& c, uint64_t cur) {
   return mn + ratio * (alpha - mn);
 }
 
-// The group of a step covers up to c.batch anchors, cut into reference batches of
-// c.rbatch; batch k of the group takes step number next_step + k (mod.rs:234 fetch_add
-// per batch) and its scheduled learning rate.
-__global__ void k_step_begin(StepConfig c, StepState* st, float lr_override) {
-  uint32_t* dt = &st->dtot[0][0];
-  for (int i = threadIdx.x; i < 4 * 2048; i += blockDim.x) dt[i] = 0u;
-  if (threadIdx.x == 0) {
-    const uint32_t sip = st->step_in_pass + 1u;  // host writes 0xFFFFFFFF at pass start
-    st->step_in_pass = sip;
-    const uint64_t base64 = (uint64_t)sip * c.batch;
-    const uint32_t base = (uint32_t)(base64 < c.n_batch_total ? base64 : c.n_batch_total);
-    st->anchor_base = base;
-    const uint32_t rem = c.n_batch_total - base;
-    const uint32_t bn = rem < c.batch ? rem : c.batch;
-    st->batch_n = bn;
-    uint32_t nb = (bn + c.rbatch - 1u) / c.rbatch;
-    if (nb > kMaxGroup) nb = kMaxGroup;
-    st->n_batches = nb;
-    const uint64_t cur = st->next_step;
-    st->next_step = cur + nb;
-    st->step0 = cur;
-    for (uint32_t k = 0; k < kMaxGroup; ++k) {
-      st->lr[k] = k < nb ? (lr_override >= 0.f ? lr_override : scheduled_lr(c, cur + k)) : 0.f;
-      // LRScheduler::exp_decay(0, noise, decay) (mod.rs:140-147, scheduler.rs:49-51); with no
-      // schedule length (explicit test steps) the sd stays at `noise`
-      float sd = 0.f;
-      if (c.noise > 1e-9f && k < nb)
-        sd = c.total_updates ? fmaxf(c.noise * powf(c.noise_decay, (float)(cur + k)), 0.f) : c.noise;
-      st->noise_sd[k] = sd;
-    }
+// The anchors of the step that starts now: the cursor step_in_pass still holds the step
+// before (k_forward / k_att_map move it on, commit_step, so every block of k_sample reads the
+// same value).
+__device__ inline void step_anchors(const StepConfig& c, const StepState* st, uint32_t* base, uint32_t* bn) {
+  const uint32_t sip = st->step_in_pass + 1u;  // host writes 0xFFFFFFFF at pass start
+  const uint64_t base64 = (uint64_t)sip * c.batch;
+  *base = (uint32_t)(base64 < c.n_batch_total ? base64 : c.n_batch_total);
+  const uint32_t rem = c.n_batch_total - *base;
+  *bn = rem < c.batch ? rem : c.batch;
+}
+
+// The step's values in StepState (one block of k_sample, nothing there reads them).  The
+// group of a step covers up to c.batch anchors, cut into reference batches of c.rbatch; batch
+// k of the group takes step number next_step + k (mod.rs:234 fetch_add per batch) and its
+// scheduled learning rate.  Lane k works out batch k's learning rate and noise.
+__device__ inline void begin_step(const StepConfig& c, StepState* st, float lr_override) {
+  uint32_t base, bn;
+  step_anchors(c, st, &base, &bn);
+  uint32_t nb = (bn + c.rbatch - 1u) / c.rbatch;
+  if (nb > kMaxGroup) nb = kMaxGroup;
+  const uint64_t cur = st->next_step;
+  const uint32_t k = threadIdx.x;
+  if (k < kMaxGroup) {
+    st->lr[k] = k < nb ? (lr_override >= 0.f ? lr_override : scheduled_lr(c, cur + k)) : 0.f;
+    // LRScheduler::exp_decay(0, noise, decay) (mod.rs:140-147, scheduler.rs:49-51); with no
+    // schedule length (explicit test steps) the sd stays at `noise`
+    float sd = 0.f;
+    if (c.noise > 1e-9f && k < nb)
+      sd = c.total_updates ? fmaxf(c.noise * powf(c.noise_decay, (float)(cur + k)), 0.f) : c.noise;
+    st->noise_sd[k] = sd;
+  } else if (k == 64u) {
     const float t = (float)st->pass + 1.0f;  // optimizer.rs:50: t = pass + 1
     st->bc1 = 1.0f - powf(0.9f, t);
     st->bc2 = 1.0f - powf(0.999f, t);
+  } else if (k == 128u) {
+    st->anchor_base = base;
+    st->batch_n = bn;
+    st->n_batches = nb;
+    st->step0 = cur;
     st->n_keys = 0u;
     st->n_real = 0u;
     st->n_unique = 0u;
@@ -484,11 +491,19 @@ __device__ inline uint32_t nth_set_bit(uint64_t m, uint32_t q) {
   return (uint32_t)__ffsll((unsigned long long)m) - 1u;
 }
 
-__global__ __launch_bounds__(256) void k_sample(StepConfig c, StepState* st) {
+// The last block begins the step (begin_step) while the others sample: they work out their
+// anchors from the cursor themselves, so the step needs no launch of its own for it.
+__global__ __launch_bounds__(256) void k_sample(StepConfig c, StepState* st, float lr_override) {
   const int lane = threadIdx.x & 63;
+  for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < 4u * 2048u; i += gridDim.x * 256u) (&st->dtot[0][0])[i] = 0u;
+  if (blockIdx.x == gridDim.x - 1u) {
+    begin_step(c, st, lr_override);
+    return;
+  }
   const uint32_t b = blockIdx.x * NW + (threadIdx.x >> 6);
   if (b >= c.batch) return;
-  const uint32_t bn = st->batch_n;
+  uint32_t abase, bn;
+  step_anchors(c, st, &abase, &bn);
   if (b >= bn) {
     if (lane == 0) {
       c.rcount[b] = 0u;
@@ -496,7 +511,7 @@ __global__ __launch_bounds__(256) void k_sample(StepConfig c, StepState* st) {
     }
     return;
   }
-  const uint32_t pos = st->anchor_base + b;
+  const uint32_t pos = abase + b;
   const uint32_t pass = st->pass;
   const uint32_t v = c.perm[pos];
   const uint64_t s0 = c.indptr[v], s1 = c.indptr[v + 1];
@@ -1005,11 +1020,14 @@ __device__ inline void forward_other_loss(const StepConfig& c, StepState* st, ui
   }
 }
 
-// 32-bit words of the float part of the forward kernel's LDS (xc, part, dist, sn),
-// rounded up to an even count so the 64-bit entry array after it is aligned.
-__host__ __device__ inline uint32_t forward_float_words(uint32_t NC, uint32_t K, uint32_t D) {
-  const uint32_t w = (NC + NW) * D + (K + 1u) + NC;
-  return (w + 1u) & ~1u;
+// Whether k_forward adds up the key offset of its example itself (and block 0 the step's key
+// count) instead of reading k_scan's: up to kForwardOffsets anchors, whose counts a block reads
+// in a few coalesced loads at its start, long before it needs the sum.  The mean model with
+// neighbour rows at fixed places; attention's block map needs the scans.  MI355X, 128 anchors:
+// k_scan took 9.4 us of a 120 us step; at 8192 anchors the blocks would read 270 MB.
+constexpr uint32_t kForwardOffsets = 2048;
+__host__ __device__ inline bool forward_offsets(const StepConfig& c) {
+  return c.model == 0 && c.batch <= kForwardOffsets && !(c.nbr_rows && (c.all_nbrs || c.pnbrs));
 }
 
 // ------------------------------------------------------------------------------------
@@ -1034,6 +1052,7 @@ __global__ __launch_bounds__(256) void k_forward(StepConfig c, StepState* st) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const uint32_t K = c.K, NC = K + 2u;
   extern __shared__ float sm[];
+  if (b == 0u && tid == 0) commit_step(st);
   float* xc = sm;                 // NC*D
   float* part = xc + NC * D;      // NW*D
   float* dist = part + NW * D;    // K+1
@@ -1050,6 +1069,36 @@ __global__ __launch_bounds__(256) void k_forward(StepConfig c, StepState* st) {
   if ((uint32_t)tid < c.ent_cap) {
     x_fs = c.ex_fs[(size_t)b * c.ent_cap + tid];
     x_fn = c.ex_fn[(size_t)b * c.ent_cap + tid];
+  }
+  // the example's key offset and the step's key count (used by the emission at the end)
+  const bool own_off = c.train && forward_offsets(c);
+  __shared__ uint32_t s_koff[NW], s_ktot[NW], s_knod[NW];
+  if (own_off) {
+    uint32_t off = 0u, tot = 0u, nodes = 0u;
+    for (uint32_t i = (uint32_t)tid; i < c.batch; i += 256u) {
+      const uint32_t x = c.rcount[i];
+      tot += x;
+      off += i < b ? x : 0u;
+      if (b == 0u && x) nodes += c.nbr_cnt[i] + K;  // an example with neighbours has rows
+    }
+    off = wave_sum_u32(off);
+    tot = wave_sum_u32(tot);
+    if (b == 0u) nodes = wave_sum_u32(nodes);
+    if (lane == 0) {
+      s_koff[w] = off;
+      s_ktot[w] = tot;
+      s_knod[w] = nodes;
+    }
+    if (b == 0u) {
+      __syncthreads();
+      if (tid == 0) {
+        const uint32_t n = (s_ktot[0] + s_ktot[1]) + (s_ktot[2] + s_ktot[3]);
+        st->n_keys = n;
+        st->stat_rows += n;
+        st->stat_nodes += (s_knod[0] + s_knod[1]) + (s_knod[2] + s_knod[3]);
+        if (n > c.key_cap) st->err = 1u;  // capacity error (checked by the host)
+      }
+    }
   }
   const uint32_t v = c.perm[st->anchor_base + b];
   const uint32_t cnt = c.nbr_cnt[b];
@@ -1069,8 +1118,11 @@ __global__ __launch_bounds__(256) void k_forward(StepConfig c, StepState* st) {
   const uint32_t k0 = (uint32_t)c.seed, k1 = (uint32_t)(c.seed >> 32);
   // read now for the key emission at the end, so no global load waits there (a load
   // after the adjoint and key stores would wait for those stores too)
-  const uint32_t kb = c.keyoff[b];
-  const bool keys_fit = st->n_keys <= c.key_cap;
+  uint32_t kb = 0u, nkeys = 0u;
+  if (!own_off) {
+    kb = c.keyoff[b];
+    nkeys = st->n_keys;
+  }
 
   __shared__ uint32_t s_wave[NW];
   __shared__ uint32_t s_np[NW];
@@ -1082,7 +1134,7 @@ __global__ __launch_bounds__(256) void k_forward(StepConfig c, StepState* st) {
   const uint32_t E = 1u + cnt + K;
   const uint32_t Re = c.rcount[b];
   const bool staged = (E <= c.ent_cap) && (Re <= c.ids_cap);
-  uint64_t* ent_fs = (uint64_t*)(sm + forward_float_words(NC, K, D));
+  uint64_t* ent_fs = (uint64_t*)(sm + c.fwd_words);
   uint64_t* ent_mask = ent_fs + c.ent_cap;  // max_features selections
   uint32_t* ent_off = (uint32_t*)(ent_mask + c.sel_cap);
   float* ent_sc = (float*)(ent_off + c.ent_cap + 1);
@@ -1439,18 +1491,26 @@ __global__ __launch_bounds__(256) void k_forward(StepConfig c, StepState* st) {
   // first-leaf hash lives in the construction / partial-sum region of the LDS, dead by
   // now; examples with more occurrences than fuse_max (5/8 of its entries) are left to
   // k_emit.
+  if (own_off) {  // the waves' sums were written before the barriers above
+    kb = (s_koff[0] + s_koff[1]) + (s_koff[2] + s_koff[3]);
+    nkeys = (s_ktot[0] + s_ktot[1]) + (s_ktot[2] + s_ktot[3]);
+    if (tid == 0) c.keyoff[b] = kb;  // for k_emit
+  }
   if (!(staged && c.fuse_emit)) return;
   if (c.grad_mode == 0 && Re > c.fuse_max) return;
-  if (!keys_fit) return;
+  if (nkeys > c.key_cap) return;
   __syncthreads();
   const uint32_t tot = ent_off[E];
   const bool first_leaf = c.grad_mode == 0;
   uint32_t* hsh = reinterpret_cast<uint32_t*>(sm);
-  const uint32_t hmask = c.fuse_hash - 1u;
+  // the example's hash: at least twice its occurrences where the region allows
+  uint32_t hsize = c.fuse_hash;
+  while (hsize > 256u && hsize / 2u >= 2u * Re) hsize /= 2u;
+  const uint32_t hmask = hsize - 1u;
   // the entry of each occurrence: one byte each (E <= 256), written entry by entry after
   // the hash where the region holds them, else a search of the entry offsets
   uint8_t* oent = reinterpret_cast<uint8_t*>(hsh + c.fuse_hash);
-  const bool ent_bytes = (size_t)c.fuse_hash * 4u + tot <= (size_t)forward_float_words(NC, K, D) * 4u;
+  const bool ent_bytes = (size_t)c.fuse_hash * 4u + tot <= (size_t)c.fwd_words * 4u;
   if (ent_bytes)
     for (uint32_t e = (uint32_t)w; e < E; e += NW)
       for (uint32_t o = ent_off[e] + (uint32_t)lane; o < ent_off[e + 1]; o += 64u) oent[o] = (uint8_t)e;
@@ -1465,7 +1525,7 @@ __global__ __launch_bounds__(256) void k_forward(StepConfig c, StepState* st) {
   };
   auto cons_of_entry = [&](uint32_t e) -> uint32_t { return e == 0u ? 0u : (e <= cnt ? 1u : 2u + (e - 1u - cnt)); };
   if (first_leaf) {
-    for (uint32_t i = tid; i < c.fuse_hash; i += blockDim.x) hsh[i] = HASH_EMPTY;
+    for (uint32_t i = tid; i < hsize; i += blockDim.x) hsh[i] = HASH_EMPTY;
     __syncthreads();
     for (uint32_t o = tid; o < tot; o += blockDim.x) {
       const uint32_t ci = cons_of_entry(entry_of(o));
@@ -3096,29 +3156,20 @@ bool row_dims_supported(int d) {
     default: return hipErrorInvalidValue;    \
   }
 
-hipError_t launch_step_begin(const StepConfig& c, StepState* st, hipStream_t s) {
-  hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(256), 0, s, c, st, -1.0f);
-  return hipGetLastError();
-}
-
-hipError_t launch_step_begin_lr(const StepConfig& c, StepState* st, float lr, hipStream_t s) {
-  hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(256), 0, s, c, st, lr);
-  return hipGetLastError();
-}
-
-hipError_t launch_sample(const StepConfig& c, StepState* st, hipStream_t s) {
-  hipLaunchKernelGGL(k_sample, dim3((c.batch + NW - 1) / NW), dim3(256), (size_t)NW * c.S * sizeof(uint32_t), s, c, st);
+hipError_t launch_sample(const StepConfig& c, StepState* st, float lr, hipStream_t s) {
+  hipLaunchKernelGGL(k_sample, dim3((c.batch + NW - 1) / NW + 1), dim3(256), (size_t)NW * c.S * sizeof(uint32_t), s, c, st,
+                     lr);
   return hipGetLastError();
 }
 
 hipError_t launch_scan(const StepConfig& c, StepState* st, hipStream_t s) {
+  if (forward_offsets(c)) return hipSuccess;  // k_forward adds up its own
   hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, c, st);
   return hipGetLastError();
 }
 
 size_t forward_lds_bytes(const StepConfig& c) {
-  const uint32_t NC = c.K + 2;
-  return (size_t)forward_float_words(NC, c.K, c.dims) * 4 + (size_t)c.ent_cap * 8 + (size_t)c.sel_cap * 12 +
+  return (size_t)c.fwd_words * 4 + (size_t)c.ent_cap * 8 + (size_t)c.sel_cap * 12 +
          (size_t)(c.ent_cap + 1) * 4 + ((size_t)c.ids_cap + ids_pad_entries(c.dims, c.bf16 != 0)) * 4;
 }
 
@@ -3146,6 +3197,7 @@ hipError_t launch_forward(const StepConfig& c, StepState* st, hipStream_t s) {
 }
 
 hipError_t launch_emit(const StepConfig& c, StepState* st, hipStream_t s) {
+  if (c.fuse_all) return hipSuccess;  // k_forward emits every example
   const size_t lds = c.grad_mode == 0 ? (size_t)c.hash_entries * sizeof(uint32_t) : 0;
   hipLaunchKernelGGL(k_emit, dim3(c.batch), dim3(256), lds, s, c, st);
   return hipGetLastError();
