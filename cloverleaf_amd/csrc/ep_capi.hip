@@ -6,6 +6,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <iterator>
 #include <mutex>
 #include <string>
 #include <type_traits>
@@ -585,8 +586,8 @@ int launch_training_step(ep_ctx* c, const ep::StepConfig& sc0, bool update, floa
 }
 
 int check_state_err(ep_ctx* c) {
-  ep::StepState hs;
-  EP_HIP(hipMemcpyAsync(&hs, c->d_state, offsetof(ep::StepState, dtot), hipMemcpyDeviceToHost, c->stream));
+  ep::StepHead hs;
+  EP_HIP(hipMemcpyAsync(&hs, c->d_state, sizeof(ep::StepHead), hipMemcpyDeviceToHost, c->stream));
   EP_HIP(hipStreamSynchronize(c->stream));
   if (hs.err) return fail(EP_ECAPACITY, "key capacity exceeded in a step");
   return EP_OK;
@@ -595,10 +596,10 @@ int check_state_err(ep_ctx* c) {
 int set_pass(ep_ctx* c, ep::StepState* st, uint32_t pass, uint64_t* next_step) {
   // pass and step_in_pass live at fixed offsets; write them with small async copies
   const uint32_t vals[2] = {pass, 0xFFFFFFFFu};
-  EP_HIP(hipMemcpyAsync((char*)st + offsetof(ep::StepState, pass), vals, sizeof(vals), hipMemcpyHostToDevice,
+  EP_HIP(hipMemcpyAsync((char*)st + offsetof(ep::StepHead, pass), vals, sizeof(vals), hipMemcpyHostToDevice,
                         c->stream));
   if (next_step)
-    EP_HIP(hipMemcpyAsync((char*)st + offsetof(ep::StepState, next_step), next_step, sizeof(uint64_t),
+    EP_HIP(hipMemcpyAsync((char*)st + offsetof(ep::StepHead, next_step), next_step, sizeof(uint64_t),
                           hipMemcpyHostToDevice, c->stream));
   EP_HIP(hipStreamSynchronize(c->stream));
   return EP_OK;
@@ -889,10 +890,12 @@ int ep_create(const ep_config* cfg, ep_ctx** out) {
   int r = c->alloc(&c->d_state, 1);
   if (r == EP_OK) r = c->alloc(&c->d_vstate, 1);
   if (r != EP_OK) { delete c; return r; }
-  ep::StepState zero{};
-  zero.next_step = 1;
-  e = hipMemcpy(c->d_state, &zero, sizeof(zero), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(c->d_vstate, &zero, sizeof(zero), hipMemcpyHostToDevice);
+  ep::StepHead head{};
+  head.next_step = 1;
+  for (ep::StepState* st : {c->d_state, c->d_vstate}) {
+    if (e == hipSuccess) e = hipMemset(st, 0, sizeof(*st));
+    if (e == hipSuccess) e = hipMemcpy(st, &head, sizeof(head), hipMemcpyHostToDevice);
+  }
   if (e != hipSuccess) { delete c; return fail(EP_EHIP, std::string("hipMemcpy: ") + hipGetErrorString(e)); }
   *out = c;
   return EP_OK;
@@ -1207,7 +1210,7 @@ int ep_learn(ep_ctx* c, ep_progress_fn progress, void* user) {
       valid_err = (float)(vs / vloss.size());
     }
     if (progress) {
-      ep::StepState hs;
+      ep::StepHead hs;
       EP_HIP(hipMemcpy(&hs, c->d_state, sizeof(hs), hipMemcpyDeviceToHost));
       progress(user, pass, hs.next_step, train_err, valid_err, hs.lr[hs.n_batches ? hs.n_batches - 1 : 0]);
     }
@@ -1366,8 +1369,8 @@ int ep_step_explicit(ep_ctx* c, const uint32_t* anchors, uint32_t n, const uint3
   int buf = 0;
   EP_TRY(launch_training_step(c, sc, false, lr, nullptr, &buf));
   EP_TRY(check_state_err(c));
-  ep::StepState hs;
-  EP_HIP(hipMemcpy(&hs, c->d_state, offsetof(ep::StepState, dtot), hipMemcpyDeviceToHost));
+  ep::StepHead hs;
+  EP_HIP(hipMemcpy(&hs, c->d_state, sizeof(ep::StepHead), hipMemcpyDeviceToHost));
   if (loss) EP_HIP(hipMemcpy(loss, sc.loss, n * sizeof(float), hipMemcpyDeviceToHost));
   if (cons)
     EP_HIP(hipMemcpy(cons, c->d_xout, (size_t)n * NC * c->cfg.dims * sizeof(float), hipMemcpyDeviceToHost));
@@ -1378,9 +1381,9 @@ int ep_step_explicit(ep_ctx* c, const uint32_t* anchors, uint32_t n, const uint3
     if (upd) {
       // the update pass re-reads the sorted keys; its long-segment lists start empty
       const uint32_t zero4[5] = {0u, 0u, 0u, 0u, 0u};  // n_unique, n_long, n_pieces, n_touched, n_short
-      static_assert(offsetof(ep::StepState, n_short) == offsetof(ep::StepState, n_unique) + 4 * sizeof(uint32_t),
+      static_assert(offsetof(ep::StepHead, n_short) == offsetof(ep::StepHead, n_unique) + 4 * sizeof(uint32_t),
                     "counter layout");
-      EP_HIP(hipMemcpy((char*)c->d_state + offsetof(ep::StepState, n_unique), zero4, sizeof(zero4),
+      EP_HIP(hipMemcpy((char*)c->d_state + offsetof(ep::StepHead, n_unique), zero4, sizeof(zero4),
                        hipMemcpyHostToDevice));
       pick_variant(c, sc);
       EP_HIP(ep::launch_scatter_sorted(sc, c->d_state, buf, c->stream));
@@ -1472,16 +1475,23 @@ int ep_step_explicit_noalloc(ep_ctx* c, const uint32_t* anchors, uint32_t n, con
   return EP_OK;
 }
 
-// Rows updated so far by the short-row kernel, and by every update path.
-static uint64_t short_rows_updated(const ep::StepState& st) {
-  uint64_t n = 0;
-  for (unsigned long long x : st.upd_short) n += x;
-  return n;
-}
-static uint64_t rows_updated(const ep::StepState& st) {
-  uint64_t n = st.stat_unique + short_rows_updated(st);
-  for (unsigned long long x : st.upd_long) n += x;
-  return n;
+// Counters of the run so far: the state's values, the rows updated by the short-row kernel
+// and by every update path.
+struct RunCounts : ep::StepHead {
+  uint64_t short_rows = 0, rows = 0;
+};
+static int read_counts(ep_ctx* c, RunCounts* out) {
+  std::vector<unsigned long long> upd(std::size(c->d_state->upd_short) + std::size(c->d_state->upd_long));
+  EP_HIP(hipMemcpy((ep::StepHead*)out, c->d_state, sizeof(ep::StepHead), hipMemcpyDeviceToHost));
+  static_assert(sizeof(ep::StepState::upd_short) == sizeof(ep::StepState::upd_long), "two counter tables, one after the other");
+  EP_HIP(hipMemcpy(upd.data(), c->d_state->upd_short, upd.size() * sizeof(upd[0]), hipMemcpyDeviceToHost));
+  out->rows = out->stat_unique;
+  out->short_rows = 0;
+  for (size_t i = 0; i < upd.size(); ++i) {
+    out->rows += upd[i];
+    if (i < upd.size() / 2) out->short_rows += upd[i];
+  }
+  return EP_OK;
 }
 
 int ep_bench_steps(ep_ctx* c, uint32_t warmup, uint32_t steps, int instrument, ep_bench_result* out) {
@@ -1518,8 +1528,8 @@ int ep_bench_steps(ep_ctx* c, uint32_t warmup, uint32_t steps, int instrument, e
   }
   EP_HIP(hipStreamSynchronize(c->stream));
   EP_TRY(check_state_err(c));
-  ep::StepState h0, h1;
-  EP_HIP(hipMemcpy(&h0, c->d_state, sizeof(h0), hipMemcpyDeviceToHost));
+  RunCounts h0, h1;
+  EP_TRY(read_counts(c, &h0));
   hipEvent_t e0, e1;
   EP_HIP(hipEventCreate(&e0));
   EP_HIP(hipEventCreate(&e1));
@@ -1539,13 +1549,13 @@ int ep_bench_steps(ep_ctx* c, uint32_t warmup, uint32_t steps, int instrument, e
   float ms = 0.f;
   EP_HIP(hipEventElapsedTime(&ms, e0, e1));
   EP_TRY(check_state_err(c));
-  EP_HIP(hipMemcpy(&h1, c->d_state, sizeof(h1), hipMemcpyDeviceToHost));
+  EP_TRY(read_counts(c, &h1));
   out->ms_total = ms;
   out->steps = steps;
   out->examples = h1.stat_examples - h0.stat_examples;
   out->rows = h1.stat_rows - h0.stat_rows;
   out->nodes = h1.stat_nodes - h0.stat_nodes;
-  out->unique_rows = rows_updated(h1) - rows_updated(h0);
+  out->unique_rows = h1.rows - h0.rows;
   out->att_items_sq = h1.stat_att_n2 - h0.stat_att_n2;
   out->att_items = h1.stat_att_n - h0.stat_att_n;
   out->seg_vpl = c->seg_vpl;
@@ -1555,15 +1565,15 @@ int ep_bench_steps(ep_ctx* c, uint32_t warmup, uint32_t steps, int instrument, e
     // per-phase timing: the same number of steps launched one by one with events
     std::vector<hipEvent_t> ev(9 * (size_t)steps);
     for (auto& e : ev) EP_HIP(hipEventCreate(&e));
-    ep::StepState g0, g1;
-    EP_HIP(hipMemcpy(&g0, c->d_state, sizeof(g0), hipMemcpyDeviceToHost));
+    RunCounts g0, g1;
+    EP_TRY(read_counts(c, &g0));
     for (uint32_t i = 0; i < steps; ++i) {
       if (in_pass == sc.steps_per_pass) EP_TRY(advance());
       else ++in_pass;
       EP_TRY(launch_training_step(c, sc, true, -1.f, &ev[9 * (size_t)i]));
     }
     EP_HIP(hipStreamSynchronize(c->stream));
-    EP_HIP(hipMemcpy(&g1, c->d_state, sizeof(g1), hipMemcpyDeviceToHost));
+    EP_TRY(read_counts(c, &g1));
     double ph[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     for (uint32_t i = 0; i < steps; ++i)
       for (int k = 0; k < 8; ++k) {
@@ -1575,7 +1585,7 @@ int ep_bench_steps(ep_ctx* c, uint32_t warmup, uint32_t steps, int instrument, e
     for (int k = 0; k < 8; ++k) out->ms_phase[k] = ph[k] / steps;
     out->ms_forward_avg = out->ms_phase[1];
     out->ms_scatter_avg = out->ms_phase[3] + out->ms_phase[4] + out->ms_phase[5] + out->ms_phase[6] + out->ms_phase[7];
-    out->short_rows = short_rows_updated(g1) - short_rows_updated(g0);
+    out->short_rows = g1.short_rows - g0.short_rows;
     out->last_long_rows = g1.n_long;
     out->last_pieces = g1.n_pieces;
     out->forward_launches = steps;

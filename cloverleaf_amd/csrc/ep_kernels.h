@@ -19,7 +19,7 @@ constexpr uint32_t kSlotMask = (1u << kSlotBatchShift) - 1u;
 // Device-resident per-step state.  Written by k_sample / k_scan / k_forward / the scatter
 // kernels; read by every kernel of the step, so one captured step graph can be
 // replayed for every batch of a pass.
-struct StepState {
+struct StepHead {
   uint64_t next_step;      // LR-schedule step counter (1-based, like the reference's AtomicUsize)
   uint64_t stat_rows;      // cumulative feature-row reads (sum of R_e)
   uint64_t stat_nodes;     // cumulative node-id reads (sampled neighbours + negatives)
@@ -45,7 +45,18 @@ struct StepState {
   float bc1, bc2;          // Adam bias corrections 1 - beta^t, t = pass + 1
   uint32_t n_real;         // non-sentinel keys (the sorted key count)
   uint32_t reg_next;       // next plan region for k_seg_update (cleared by k_seg_plan)
+};
+
+// Sort grids of up to kSortGroups x kSortGroupBlocks blocks keep digit totals per group of
+// blocks (see k_rs_scatter).
+constexpr uint32_t kSortGroups = 16u, kSortGroupBlocks = 16u;
+
+// The device's state: the values above (what the host reads back) and the tables.
+struct StepState : StepHead {
   uint32_t dtot[4][2048];  // radix-sort digit totals, one row per sort pass (<= 11-bit digits)
+  // digit totals of groups of sort blocks, kSortGroups tables per pass (at most 2 passes of
+  // 11-bit or 3 of 9-bit digits)
+  uint32_t dgrp[2 * kSortGroups * 2048];
   // cumulative rows updated, one slot per block of the row kernels: by the short-row kernel,
   // and by the medium- and long-row kernels (stat_unique: by the atomic path)
   unsigned long long upd_short[2048], upd_long[2048];
@@ -169,6 +180,8 @@ struct StepConfig {
   uint32_t key_cap;
   uint32_t* ghist;         // [2048 * sort_grid]
   int sort_grid;
+  int sort_groups;         // k_sample clears dgrp (1) or dtot (0), sort_totals words of it (set by
+  uint32_t sort_totals;    // launch_sample)
   // scatter (sort path)
   float* G;                // [key_cap*D] compact gradient rows (bounded by unique count)
   uint32_t* ufeat;         // [key_cap]

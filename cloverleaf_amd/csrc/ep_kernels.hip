@@ -495,7 +495,9 @@ __device__ inline uint32_t nth_set_bit(uint64_t m, uint32_t q) {
 // anchors from the cursor themselves, so the step needs no launch of its own for it.
 __global__ __launch_bounds__(256) void k_sample(StepConfig c, StepState* st, float lr_override) {
   const int lane = threadIdx.x & 63;
-  for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < 4u * 2048u; i += gridDim.x * 256u) (&st->dtot[0][0])[i] = 0u;
+  // the sort's totals: of the whole grid (k_rs_scan's) or of its groups, whichever it uses
+  uint32_t* totals = c.sort_groups ? st->dgrp : &st->dtot[0][0];
+  for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < c.sort_totals; i += gridDim.x * 256u) totals[i] = 0u;
   if (blockIdx.x == gridDim.x - 1u) {
     begin_step(c, st, lr_override);
     return;
@@ -1694,7 +1696,9 @@ __device__ inline uint64_t digit_peers(bool act, uint32_t d) {
 
 // Pass 0 reads the emitted keys (st->n_keys, sentinels included) and drops the sentinels;
 // later passes read the st->n_real compacted keys.
-template <int RB>
+// GROUPS: also the totals of groups of kSortGroupBlocks blocks, for a k_rs_scatter that works
+// out its digit bases itself.
+template <int RB, bool GROUPS>
 __global__ __launch_bounds__(256) void k_rs_hist(const uint32_t* __restrict__ kin, StepState* st, uint32_t* ghist,
                                                  int pass, int shift, int G, uint32_t sent) {
   constexpr uint32_t BINS = 1u << RB, MASK = BINS - 1u;
@@ -1702,6 +1706,7 @@ __global__ __launch_bounds__(256) void k_rs_hist(const uint32_t* __restrict__ ki
   const int tid = threadIdx.x, lane = tid & 63;
   uint32_t lo, hi;
   block_range(pass == 0 ? st->n_keys : st->n_real, G, blockIdx.x, &lo, &hi);
+  if (GROUPS && lo >= hi) return;  // k_rs_scatter reads the counts of blocks with elements only
   for (uint32_t d = tid; d < BINS; d += 256u) h[d] = 0u;
   __syncthreads();
   for (uint32_t t0 = lo; t0 < hi; t0 += 256u * RS_ITEMS) {
@@ -1730,10 +1735,18 @@ __global__ __launch_bounds__(256) void k_rs_hist(const uint32_t* __restrict__ ki
   __syncthreads();
   for (uint32_t d = tid; d < BINS; d += 256u) {
     ghist[(size_t)blockIdx.x * BINS + d] = h[d];  // block-major: coalesced
-    if (h[d]) atomicAdd(&st->dtot[pass][d], h[d]);
+    uint32_t* tot = GROUPS ? &st->dgrp[((uint32_t)pass * kSortGroups + blockIdx.x / kSortGroupBlocks) * BINS + d]
+                           : &st->dtot[pass][d];
+    if (h[d]) atomicAdd(tot, h[d]);
   }
 }
 
+// Grids of up to kSortGroups x kSortGroupBlocks blocks (steps of up to 2M keys at capacity):
+// every scatter block adds up its bases from the group totals and its group's counts, at most
+// 32 coalesced reads per digit, instead of a k_rs_scan launch between the two kernels (6.6 of
+// 17 us of a pass at 16k keys on MI355X; at 2048 blocks the reads would cost what the scan
+// does).
+//
 // Turns the block-major counts into scatter bases: base(blk, d) = sum_{d' < d} total(d')
 // + sum_{b < blk} count(b, d).  One wave per digit; lane l owns G/64 consecutive source
 // blocks (their loads are independent), then a wave scan.
@@ -1775,7 +1788,7 @@ __global__ __launch_bounds__(256) void k_rs_scan(uint32_t* ghist, StepState* st,
 // and blocks follow each other through the per-block digit bases.
 static constexpr int RS_SCATTER_ITEMS = 16;
 
-template <int RB>
+template <int RB, bool GROUPS>
 __global__ __launch_bounds__(256) void k_rs_scatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
                                                     uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
                                                     StepState* st, const uint32_t* __restrict__ ghist, int pass,
@@ -1793,24 +1806,60 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const uint32_t* __restrict__
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   uint32_t lo, hi;
   block_range(pass == 0 ? st->n_keys : st->n_real, G, blockIdx.x, &lo, &hi);
+  if (GROUPS && lo >= hi) return;
+  if constexpr (GROUPS) {
+    // base(d) = totals of the smaller digits + counts of d in the blocks before this one:
+    // thread tid owns digits [tid*DPT, tid*DPT + DPT)
+    const uint32_t grp = blockIdx.x / kSortGroupBlocks;
+    const uint32_t* gs = st->dgrp + (uint32_t)pass * kSortGroups * BINS;
+    uint32_t bef[DPT], tot[DPT], tsum = 0u;
+#pragma unroll
+    for (uint32_t j = 0; j < DPT; ++j) {
+      const uint32_t d = (uint32_t)tid * DPT + j;
+      bef[j] = tot[j] = 0u;
+      if (d < BINS) {
+#pragma unroll
+        for (uint32_t q = 0; q < kSortGroups; ++q) {
+          const uint32_t x = gs[q * BINS + d];
+          tot[j] += x;
+          bef[j] += q < grp ? x : 0u;
+        }
+        for (uint32_t b = grp * kSortGroupBlocks; b < blockIdx.x; ++b) bef[j] += ghist[(size_t)b * BINS + d];
+      }
+      tsum += tot[j];
+    }
+    uint32_t all = 0u;
+    uint32_t start = block_exclusive_scan(tsum, s_wave, &all);
+    if (blockIdx.x == 0u && tid == 0 && pass == 0) st->n_real = all;
+#pragma unroll
+    for (uint32_t j = 0; j < DPT; ++j) {
+      const uint32_t d = (uint32_t)tid * DPT + j;
+      if (d < BINS) run[d] = start + bef[j];
+      start += tot[j];
+    }
+  }
   for (uint32_t d = tid; d < BINS; d += 256u) {
-    run[d] = ghist[(size_t)blockIdx.x * BINS + d];
+    if constexpr (!GROUPS) run[d] = ghist[(size_t)blockIdx.x * BINS + d];
 #pragma unroll
     for (int q = 0; q < NW; ++q) wcnt[q][d] = 0u;
   }
   __syncthreads();
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  // a block of a small step holds less than a tile: its waves share what there is
+  const uint32_t span = GROUPS ? (min(hi - lo, TILE) + 255u) / 256u * 64u : WSPAN;
   for (uint32_t t0 = lo; t0 < hi; t0 += TILE) {
     uint32_t k[IT], val[IT], rk[IT];
 #pragma unroll
     for (int q = 0; q < IT; ++q) {
-      const uint32_t i = t0 + (uint32_t)w * WSPAN + (uint32_t)q * 64u + (uint32_t)lane;
-      k[q] = i < hi ? kin[i] : sent;  // sent: inactive (pass 0 drops the sentinels)
-      val[q] = i < hi ? vin[i] : 0u;
+      const uint32_t i = t0 + (uint32_t)w * span + (uint32_t)q * 64u + (uint32_t)lane;
+      const bool in = (!GROUPS || (uint32_t)q * 64u < span) && i < hi;
+      k[q] = in ? kin[i] : sent;  // sent: inactive (pass 0 drops the sentinels)
+      val[q] = in ? vin[i] : 0u;
     }
     // ranks within the wave's quarter: count of earlier elements with the same digit
 #pragma unroll
     for (int q = 0; q < IT; ++q) {
+      if (GROUPS && (uint32_t)q * 64u >= span) break;
       const bool act = k[q] != sent;
       const uint32_t d = (k[q] >> shift) & MASK;
       // the lanes sharing this lane's digit: all active lanes when the wave holds one digit
@@ -3156,7 +3205,18 @@ bool row_dims_supported(int d) {
     default: return hipErrorInvalidValue;    \
   }
 
-hipError_t launch_sample(const StepConfig& c, StepState* st, float lr, hipStream_t s) {
+// Digit plan: passes = ceil(bits / 11), RB = ceil(bits / passes).
+static void radix_plan(int bits, int* passes, int* rb) {
+  *passes = (bits + 10) / 11;
+  *rb = (bits + *passes - 1) / *passes;
+}
+
+hipError_t launch_sample(const StepConfig& c0, StepState* st, float lr, hipStream_t s) {
+  StepConfig c = c0;
+  int passes, rb;
+  radix_plan(c.sort_bits, &passes, &rb);
+  c.sort_groups = c.sort_grid <= (int)(kSortGroups * kSortGroupBlocks);
+  c.sort_totals = !c.train ? 0u : c.sort_groups ? ((uint32_t)passes * kSortGroups) << rb : 4u * 2048u;
   hipLaunchKernelGGL(k_sample, dim3((c.batch + NW - 1) / NW + 1), dim3(256), (size_t)NW * c.S * sizeof(uint32_t), s, c, st,
                      lr);
   return hipGetLastError();
@@ -3203,12 +3263,6 @@ hipError_t launch_emit(const StepConfig& c, StepState* st, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Digit plan: passes = ceil(bits / 11), RB = ceil(bits / passes).
-static void radix_plan(int bits, int* passes, int* rb) {
-  *passes = (bits + 10) / 11;
-  *rb = (bits + *passes - 1) / *passes;
-}
-
 // Blocks of 256 threads of kernel K resident on the current device at once, at most cap.
 // The three runtime queries cost more than a launch, so the answer (a property of the built
 // kernel and the device model) is kept per kernel and device.
@@ -3228,22 +3282,30 @@ static int resident_blocks(int cap) {
   return n < cap ? n : cap;
 }
 
-template <int RB>
-static void launch_sort_rb(const StepConfig& c, StepState* st, hipStream_t s, int passes, int* cur) {
+template <int RB, bool GROUPS>
+static void launch_sort_passes(const StepConfig& c, StepState* st, hipStream_t s, int passes, int* cur) {
   // whole rounds of resident scatter blocks (at 9-bit digits its tile and counters take
   // 44 KB of LDS, three blocks per CU): a last, partial round would leave part of the
   // device idle; the three kernels of a pass share the block partition
-  const int res = resident_blocks<k_rs_scatter<RB>>(c.sort_grid);
+  const int res = resident_blocks<k_rs_scatter<RB, GROUPS>>(c.sort_grid);
   const int G = res < c.sort_grid ? (c.sort_grid / res) * res : c.sort_grid;
   for (int p = 0; p < passes; ++p) {
     const int shift = p * RB;
-    hipLaunchKernelGGL((k_rs_hist<RB>), dim3(G), dim3(256), 0, s, c.keys[*cur], st, c.ghist, p, shift, G,
+    hipLaunchKernelGGL((k_rs_hist<RB, GROUPS>), dim3(G), dim3(256), 0, s, c.keys[*cur], st, c.ghist, p, shift, G,
                        c.sentinel);
-    hipLaunchKernelGGL((k_rs_scan<RB>), dim3(((1u << RB) + NW - 1u) / NW), dim3(256), 0, s, c.ghist, st, p, G);
-    hipLaunchKernelGGL((k_rs_scatter<RB>), dim3(G), dim3(256), 0, s, c.keys[*cur], c.slots[*cur], c.keys[1 - *cur],
-                       c.slots[1 - *cur], st, c.ghist, p, shift, G, c.sentinel);
+    if constexpr (!GROUPS)
+      hipLaunchKernelGGL((k_rs_scan<RB>), dim3(((1u << RB) + NW - 1u) / NW), dim3(256), 0, s, c.ghist, st, p, G);
+    hipLaunchKernelGGL((k_rs_scatter<RB, GROUPS>), dim3(G), dim3(256), 0, s, c.keys[*cur], c.slots[*cur],
+                       c.keys[1 - *cur], c.slots[1 - *cur], st, c.ghist, p, shift, G, c.sentinel);
     *cur = 1 - *cur;
   }
+}
+
+template <int RB>
+static void launch_sort_rb(const StepConfig& c, StepState* st, hipStream_t s, int passes, int* cur) {
+  static_assert(kSortGroups << RB <= sizeof(StepState::dgrp) / sizeof(uint32_t) / (RB <= 9 ? 3 : 2), "a table per pass");
+  if (c.sort_grid <= (int)(kSortGroups * kSortGroupBlocks)) launch_sort_passes<RB, true>(c, st, s, passes, cur);
+  else launch_sort_passes<RB, false>(c, st, s, passes, cur);
 }
 
 hipError_t launch_sort(const StepConfig& c, StepState* st, hipStream_t s, int* out_buf) {
