@@ -544,7 +544,8 @@ void refresh_base(ep_ctx* c) {
 // results).
 void pick_variant(const ep_ctx* c, ep::StepConfig& sc) {
   if (sc.fwd_x == 0) sc.fwd_x = c->fwd_x ? c->fwd_x : 1;
-  if (sc.seg_vpl != 0) return;
+  if (sc.seg_vpl != 0) return;  // the tuner's candidate
+  sc.any_tile = c->cfg.seg_vpl == 0 ? 1 : 0;
   sc.seg_vpl = c->seg_vpl ? c->seg_vpl : 4;
   sc.seg_unroll = c->seg_vpl ? c->seg_unroll : 8;
 }

@@ -227,6 +227,7 @@ struct StepConfig {
                            // ufeat = row | batch << 27
   int unique_grid;         // grid size for the persistent row kernels
   int seg_vpl;             // k_seg_adam values per lane (4, 8, 16; chosen by the tuner)
+  int any_tile;            // 1: the tile was not asked for by name and is not being tuned
   int seg_unroll;          // k_seg_adam adjoint rows in flight per lane group (tuned)
   int fwd_x;               // k_forward rows-in-flight multiplier of the wide gathers: 1 or 2 (tuned)
   // Attention model (model = 1): rows are [Q_1..Q_H | K_1..K_H | V_1..V_H], dims =

@@ -1947,17 +1947,31 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const uint32_t* __restrict__
 // quarter of their instructions (the update applies one Adam step per batch of the
 // group to every value of every touched row).
 // ------------------------------------------------------------------------------------
+// The fused multiply-adds are spelled out, so that the rounding of a row does not hang on what
+// the compiler contracts in one kernel or another: adam_math (short rows, atomic path) rounds
+// the decayed moment before the fused add, adam_math_run (medium and long rows) the new
+// gradient's part.
+__device__ inline void adam_step(float& th, float m, float v, float lr, float ibc1, float ibc2) {
+  const float den = __builtin_amdgcn_sqrtf(v * ibc2) + 1e-8f;
+  th = __builtin_fmaf(-(lr * (m * ibc1)), __builtin_amdgcn_rcpf(den), th);
+}
 __device__ inline void adam_math(float& th, float& m, float& v, float g, float lr, float ibc1, float ibc2) {
-  const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-  m = b1 * m + (1.0f - b1) * g;
-  v = b2 * v + (1.0f - b2) * (g * g);
-  const float den = __builtin_amdgcn_sqrtf(v * ibc2) + eps;
-  th -= lr * (m * ibc1) * __builtin_amdgcn_rcpf(den);
+  const float b1 = 0.9f, b2 = 0.999f;
+  m = __builtin_fmaf(1.0f - b1, g, b1 * m);
+  v = __builtin_fmaf(1.0f - b2, g * g, b2 * v);
+  adam_step(th, m, v, lr, ibc1, ibc2);
+}
+__device__ inline void adam_math_run(float& th, float& m, float& v, float g, float lr, float ibc1, float ibc2) {
+  const float b1 = 0.9f, b2 = 0.999f;
+  m = __builtin_fmaf(b1, m, (1.0f - b1) * g);
+  v = __builtin_fmaf(b2, v, (1.0f - b2) * (g * g));
+  adam_step(th, m, v, lr, ibc1, ibc2);
 }
 
 // k_seg_update's units (see there): a region's rows go to at most kUpdSplitMax units, about
 // kUpdUnitsPerWave per wave of the grid.
 static constexpr uint32_t kUpdSplitMax = 16, kUpdUnitsPerWave = 2;
+static constexpr uint32_t kRowsOneLaunch = 1u << 21;  // k_rows: keys at capacity
 
 // Per-step scalars of the update, read once per kernel (before any store, so the
 // compiler keeps them in registers instead of reloading them after each store).
@@ -2362,8 +2376,10 @@ __device__ inline void count_rows(unsigned long long* slots, uint32_t x) {
 // the fastest.
 // NZ: the gradient-noise path (noise > 0), built for one tile per width only: its
 // Philox and transcendental code would raise every tile's VGPRs (and cut its waves).
-template <int D, int VPL, int U, bool H, bool NZ = false>
-__global__ __launch_bounds__(256) void k_seg_update(StepConfig c, StepState* st, const uint32_t* __restrict__ Ss) {
+// blk of grid blocks run the short rows (the whole grid of k_seg_update, part of k_rows').
+template <int D, int VPL, int U, bool H, bool NZ>
+__device__ inline void short_rows(const StepConfig& c, StepState* st, const uint32_t* __restrict__ Ss, uint32_t blk,
+                                  uint32_t grid) {
   static_assert(D % VPL == 0 && VPL % 4 == 0 && D / VPL <= 64, "float4 lane slices");
   constexpr int L = D / VPL;      // lanes per row
   constexpr int G = 64 / L;       // rows in flight per wave
@@ -2393,14 +2409,14 @@ __global__ __launch_bounds__(256) void k_seg_update(StepConfig c, StepState* st,
   // groups sub, sub + split, ... of region u % nreg, sub = u / nreg) and wave gw takes units
   // gw, gw + waves, ...: no atomics, and no wave holds the up to 64 rows that start in one
   // chunk of cold keys while others hold none.
-  const uint32_t nwv = gridDim.x * NW;
+  const uint32_t nwv = grid * NW;
   const bool queued = nreg > nwv;
   uint32_t split = 1u;
   if (!queued)
     while (split < kUpdSplitMax && nreg * split < kUpdUnitsPerWave * nwv) split *= 2u;
   const uint32_t units = nreg * split;
   const uint32_t stride = (uint32_t)G * split;  // rows between two of a lane group's
-  for (uint32_t unit = blockIdx.x * NW + (uint32_t)(tid >> 6);;) {
+  for (uint32_t unit = blk * NW + (uint32_t)(tid >> 6);;) {
     if (unit >= units) break;
     const uint32_t reg = queued ? unit : unit % nreg;
     const uint32_t first = queued ? 0u : unit / nreg * (uint32_t)G;  // the unit's first row group
@@ -2615,6 +2631,11 @@ __global__ __launch_bounds__(256) void k_seg_update(StepConfig c, StepState* st,
   count_rows(st->upd_short, done);
 }
 
+template <int D, int VPL, int U, bool H, bool NZ = false>
+__global__ __launch_bounds__(256) void k_seg_update(StepConfig c, StepState* st, const uint32_t* __restrict__ Ss) {
+  short_rows<D, VPL, U, H, NZ>(c, st, Ss, blockIdx.x, gridDim.x);
+}
+
 // Loads row f's optimizer operands (whole-wave slice layout).
 template <int D>
 __device__ inline void load_row_state(const StepConfig& c, uint32_t f, int lane, float (&th)[RowShape<D>::PL],
@@ -2671,7 +2692,7 @@ __device__ inline bool apply_run(const StepConfig& c, StepState* st, const StepS
   for (int q = 0; q < PL; ++q) bad |= (base + q < D) && isnan(acc[q]);
   if (wave_any(bad)) return false;
 #pragma unroll
-  for (int q = 0; q < PL; ++q) adam_math(th[q], m[q], v[q], acc[q], lr, sv.ibc1, sv.ibc2);
+  for (int q = 0; q < PL; ++q) adam_math_run(th[q], m[q], v[q], acc[q], lr, sv.ibc1, sv.ibc2);
   return true;
 }
 
@@ -2696,22 +2717,15 @@ __device__ inline void add_rows_tree(float (&acc)[PL], float (&r)[U][PL], uint32
 }
 
 // Partial sums of the pieces of long rows (each piece: <= kPieceEntries entries of one
-// run), then the medium rows of this wave's plan region: one wave per row (<= 128
-// entries), its runs reduced from the adjoint rows and applied in batch order.
+// run), by block blk of grid.
 template <int D, bool H>
-__global__ __launch_bounds__(256) void k_pieces(StepConfig c, StepState* st, const uint32_t* __restrict__ Ks,
-                                                const uint32_t* __restrict__ Ss) {
+__device__ inline void piece_sums(const StepConfig& c, StepState* st, const uint32_t* __restrict__ Ss, uint32_t blk,
+                                  uint32_t grid) {
   constexpr int PL = RowShape<D>::PL;
   constexpr int U = SR_UNROLL;
-  __shared__ float s_lr[kMaxGroup], s_sd[kMaxGroup];
   const int lane = threadIdx.x & 63;
-  const uint32_t gw = blockIdx.x * NW + (threadIdx.x >> 6);
-  const uint32_t nwaves = gridDim.x * NW;
-  if (threadIdx.x < kMaxGroup) {
-    s_lr[threadIdx.x] = st->lr[threadIdx.x];
-    s_sd[threadIdx.x] = st->noise_sd[threadIdx.x];
-  }
-  __syncthreads();
+  const uint32_t gw = blk * NW + (threadIdx.x >> 6);
+  const uint32_t nwaves = grid * NW;
   const uint32_t np = st->n_pieces < c.piece_cap ? st->n_pieces : c.piece_cap;
   // Batch by batch: a piece reads adjoint rows of its batch only, so every wave working
   // on the same batch keeps the rows being read within one batch's share of the adjoint
@@ -2741,7 +2755,24 @@ __global__ __launch_bounds__(256) void k_pieces(StepConfig c, StepState* st, con
     }
     store_slice<D>(c.part + (size_t)gp * D, lane, acc);
   }
-  // medium rows of the plan regions gw, gw + nwaves, ...
+}
+
+// The medium rows of the plan regions, dealt to the waves of grid blocks: one wave per row
+// (<= 128 entries), its runs reduced from the adjoint rows and applied in batch order.
+template <int D, bool H>
+__device__ inline void medium_rows(const StepConfig& c, StepState* st, const uint32_t* __restrict__ Ks,
+                                   const uint32_t* __restrict__ Ss, uint32_t blk, uint32_t grid) {
+  constexpr int PL = RowShape<D>::PL;
+  constexpr int U = SR_UNROLL;
+  __shared__ float s_lr[kMaxGroup], s_sd[kMaxGroup];
+  const int lane = threadIdx.x & 63;
+  const uint32_t gw = blk * NW + (threadIdx.x >> 6);
+  const uint32_t nwaves = grid * NW;
+  if (threadIdx.x < kMaxGroup) {
+    s_lr[threadIdx.x] = st->lr[threadIdx.x];
+    s_sd[threadIdx.x] = st->noise_sd[threadIdx.x];
+  }
+  __syncthreads();
   const uint32_t n = st->n_keys <= c.key_cap ? st->n_real : 0u;
   const uint32_t nchunks = (n + 63u) / 64u;
   const uint32_t cpr = (nchunks + c.n_regions - 1u) / c.n_regions;
@@ -2800,6 +2831,29 @@ __global__ __launch_bounds__(256) void k_pieces(StepConfig c, StepState* st, con
     }
   }
   count_rows(st->upd_long, lane == 0 ? done : 0u);
+}
+
+template <int D, bool H>
+__global__ __launch_bounds__(256) void k_pieces(StepConfig c, StepState* st, const uint32_t* __restrict__ Ks,
+                                                const uint32_t* __restrict__ Ss) {
+  piece_sums<D, H>(c, st, Ss, blockIdx.x, gridDim.x);
+  medium_rows<D, H>(c, st, Ks, Ss, blockIdx.x, gridDim.x);
+}
+
+// The segment tile of a launch that has no tuned one.
+template <int D> constexpr int kTileV = (D % 4 == 0 && D / 4 <= 64) ? 4 : 16;
+template <int D> constexpr int kTileU = kTileV<D> == 4 ? 8 : 2;
+
+// Small steps: the pieces, the medium rows and the short rows are different rows, so blocks
+// of one launch take them side by side; one after the other each is a chain of loads on a device
+// mostly idle (see rows_in_one_launch for both times).
+template <int D, bool H>
+__global__ __launch_bounds__(256) void k_rows(StepConfig c, StepState* st, const uint32_t* __restrict__ Ks,
+                                              const uint32_t* __restrict__ Ss, uint32_t npiece, uint32_t nmed) {
+  const uint32_t b = blockIdx.x;
+  if (b < nmed) medium_rows<D, H>(c, st, Ks, Ss, b, nmed);
+  else if (b < nmed + npiece) piece_sums<D, H>(c, st, Ss, b - nmed, npiece);
+  else short_rows<D, kTileV<D>, kTileU<D>, H, false>(c, st, Ss, b - nmed - npiece, gridDim.x - nmed - npiece);
 }
 
 // One wave per long row: loads theta/m/v once, adds the pieces of each run in order and
@@ -3350,6 +3404,15 @@ bool seg_variant_supported(int d, int vpl, int unroll) {
   return unroll == 8 / nq || unroll == 16 / nq || (nq <= 2 && unroll == 4 / nq);
 }
 
+// Steps of few enough keys for one launch of the row kernels (k_rows); a tile asked for by
+// name, the tuner's candidates and gradient noise have k_seg_update instances of their own.
+// MI355X, one launch against two: 16k keys of D = 64 11.8 against 21.2 us, 0.4M keys of
+// D = 128 45 against 60; at D = 768 (256 VGPRs, one wave per SIMD for every role) it gains
+// nothing, so the attention widths past 256 keep two.
+static bool rows_in_one_launch(const StepConfig& c) {
+  return c.any_tile && c.dims <= 256 && c.key_cap <= kRowsOneLaunch && !(c.noise > 1e-9f);
+}
+
 template <int D, int VPL, int U, bool H>
 static bool try_seg_update(const StepConfig& c, StepState* st, int buf, hipStream_t s, int grid) {
   if constexpr (D % VPL == 0 && D / VPL <= 64) {
@@ -3389,6 +3452,20 @@ static void launch_row_kernels(const StepConfig& c, StepState* st, int buf, hipS
   // grids that the step's largest key count can fill: blocks for `per` waves per 64-key chunk
   const uint64_t chunks = ((uint64_t)c.key_cap + 63u) / 64u;
   auto wave_grid = [&](uint64_t per) { return (int)std::min<uint64_t>(c.unique_grid, (chunks * per + NW - 1u) / NW); };
+  const int lgrid = resident_blocks<k_long_combine<D, H>>(wave_grid(1));
+  if (D <= 256 && rows_in_one_launch(c)) {
+    // medium rows: a wave per chunk; pieces: two; short rows: the rest of unique_grid blocks
+    const uint32_t nmed = (uint32_t)std::min(wave_grid(1), c.unique_grid / 8);
+    const uint32_t npiece = (uint32_t)std::min(wave_grid(2), c.unique_grid / 4);
+    const uint32_t nshort = (uint32_t)std::min<uint64_t>(wave_grid(kUpdSplitMax), c.unique_grid - nmed - npiece);
+    if constexpr (D <= 256) hipLaunchKernelGGL((k_rows<D, H>), dim3(nmed + npiece + nshort), dim3(256), 0, s, c, st, c.keys[buf], c.slots[buf],
+                       npiece, nmed);
+    if (ev) (void)hipEventRecord(ev[1], s);
+    if (ev) (void)hipEventRecord(ev[2], s);
+    hipLaunchKernelGGL((k_long_combine<D, H>), dim3(lgrid), dim3(256), 0, s, c, st, c.keys[buf], c.slots[buf]);
+    if (ev) (void)hipEventRecord(ev[3], s);
+    return;
+  }
   launch_seg_update_variant<D, H>(c, st, buf, s, wave_grid(kUpdSplitMax));
   if (ev) (void)hipEventRecord(ev[1], s);
   // k_pieces sweeps the pieces batch by batch: one round of resident blocks keeps every
@@ -3397,7 +3474,6 @@ static void launch_row_kernels(const StepConfig& c, StepState* st, int buf, hipS
   hipLaunchKernelGGL((k_pieces<D, H>), dim3(pgrid), dim3(256), 0, s, c, st, c.keys[buf], c.slots[buf]);
   if (ev) (void)hipEventRecord(ev[2], s);
   // hot rows dealt to one round of resident blocks: no late blocks holding the last rows
-  const int lgrid = resident_blocks<k_long_combine<D, H>>(wave_grid(1));
   hipLaunchKernelGGL((k_long_combine<D, H>), dim3(lgrid), dim3(256), 0, s, c, st, c.keys[buf], c.slots[buf]);
   if (ev) (void)hipEventRecord(ev[3], s);
 }
