@@ -239,36 +239,32 @@ __device__ inline void store_slice_f16(uint16_t* __restrict__ row, int lane, con
   }
 }
 
-// v = mul * row slice (zero outside the row)
+// Row slice as stored, two values per word (zero outside the row), and one of its values.
 template <int D>
-__device__ inline void load_slice_f16(const uint16_t* __restrict__ row, int lane, float (&v)[RowShape<D>::PL],
-                                      float mul) {
+__device__ inline void load_packed_f16(const uint16_t* __restrict__ row, int lane,
+                                       uint32_t (&w)[(RowShape<D>::PL + 1) / 2]) {
   constexpr int PL = RowShape<D>::PL;
   const int base = lane * PL;
   if constexpr (PL % 4 == 0 && D % PL == 0) {
-    if (base < D) {
 #pragma unroll
-      for (int k = 0; k < PL; k += 4) {
-        const uint2 t = *reinterpret_cast<const uint2*>(row + base + k);
-        v[k] = mul * f16_to_f32((uint16_t)(t.x & 0xffffu));
-        v[k + 1] = mul * f16_to_f32((uint16_t)(t.x >> 16));
-        v[k + 2] = mul * f16_to_f32((uint16_t)(t.y & 0xffffu));
-        v[k + 3] = mul * f16_to_f32((uint16_t)(t.y >> 16));
-      }
-    } else {
-#pragma unroll
-      for (int k = 0; k < PL; ++k) v[k] = 0.f;
+    for (int k = 0; k < PL; k += 4) {
+      const uint2 t = base < D ? *reinterpret_cast<const uint2*>(row + base + k) : make_uint2(0u, 0u);
+      w[k / 2] = t.x;
+      w[k / 2 + 1] = t.y;
     }
   } else if constexpr (PL == 2 && D % 2 == 0) {
-    if (base < D) {
-      const uint32_t t = *reinterpret_cast<const uint32_t*>(row + base);
-      v[0] = mul * f16_to_f32((uint16_t)(t & 0xffffu));
-      v[1] = mul * f16_to_f32((uint16_t)(t >> 16));
-    } else { v[0] = v[1] = 0.f; }
+    w[0] = base < D ? *reinterpret_cast<const uint32_t*>(row + base) : 0u;
   } else {
 #pragma unroll
-    for (int j = 0; j < PL; ++j) v[j] = (base + j < D) ? mul * f16_to_f32(row[base + j]) : 0.f;
+    for (int j = 0; j < PL; j += 2) {
+      w[j / 2] = base + j < D ? row[base + j] : 0u;
+      if (j + 1 < PL && base + j + 1 < D) w[j / 2] |= (uint32_t)row[base + j + 1] << 16;
+    }
   }
+}
+template <int N>
+__device__ inline float packed_half(const uint32_t (&w)[N], int q) {
+  return f16_to_f32((uint16_t)((q & 1) ? w[q / 2] >> 16 : w[q / 2] & 0xffffu));
 }
 
 // ------------------------------------------------------------------------------------

@@ -74,12 +74,6 @@ __device__ inline void store_adj_row(const StepConfig& c, size_t slot, int lane,
   }
 }
 
-template <int D, bool H>
-__device__ inline void load_adj_row(const StepConfig& c, size_t slot, int lane, float (&r)[RowShape<D>::PL]) {
-  if constexpr (H) load_slice_f16<D>(c.adjh + slot * D, lane, r, c.ascale[slot]);
-  else load_slice<D>(c.adj + slot * D, lane, r);
-}
-
 // First index i in [lo, hi) with K[i] >= x (hi if none), K sorted; 64-ary search by
 // the whole wave.
 __device__ inline uint32_t wave_lower_bound(const uint32_t* __restrict__ K, uint32_t lo, uint32_t hi, uint32_t x) {
@@ -2702,10 +2696,12 @@ __device__ inline bool apply_run(const StepConfig& c, StepState* st, const StepS
 template <int U, int PL>
 __device__ inline void add_rows_tree(float (&acc)[PL], float (&r)[U][PL], uint32_t n) {
   static_assert((U & (U - 1)) == 0, "U is a power of two");
+  if (n < (uint32_t)U) {
 #pragma unroll
-  for (int u = 0; u < U; ++u)
+    for (int u = 0; u < U; ++u)
 #pragma unroll
-    for (int q = 0; q < PL; ++q) r[u][q] = (uint32_t)u < n ? r[u][q] : 0.f;
+      for (int q = 0; q < PL; ++q) r[u][q] = (uint32_t)u < n ? r[u][q] : 0.f;
+  }
 #pragma unroll
   for (int w = 1; w < U; w *= 2)
 #pragma unroll
@@ -2716,6 +2712,64 @@ __device__ inline void add_rows_tree(float (&acc)[PL], float (&r)[U][PL], uint32
   for (int q = 0; q < PL; ++q) acc[q] += r[0][q];
 }
 
+__device__ inline uint32_t wave_uniform(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
+__device__ inline uint32_t lane_value(uint32_t x, uint32_t lane) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)x, (int)lane);
+}
+
+// Up to 64 adjoint rows named by lane: lane i holds row i's slot and, for FP16 rows, its scale.
+template <bool H>
+struct RowNames {
+  uint32_t slot;
+  float scale;
+};
+template <bool H>
+__device__ inline RowNames<H> row_names(const StepConfig& c, uint32_t slot) {
+  if constexpr (H) return RowNames<H>{slot, c.ascale[slot]};
+  else return RowNames<H>{slot, 1.f};
+}
+
+// acc += rows [t0, t0 + min(U, n)) of the names (wave-uniform t0 and n >= 1), as add_rows_tree
+// adds them.  The names are read lane by lane into scalar registers, so a row's address is
+// scalar arithmetic (a shuffle goes through the LDS and leaves it to the vector ALUs), and FP16
+// rows stay packed until the tree's first level, where one mixed-precision multiply-add takes
+// a half, its row's scale and the partner's product: the scales are powers of two, so the
+// products are exact and the sum is rounded once, as an add of widened rows is.  At D = 256
+// about 9 vector instructions per row against 30.  Pieces of the 10M-node shape (FP32 rows of
+// 256) 494 -> 410 us, of the 50M-node shape (FP16 rows) 4.94 -> 4.57 ms, there at 6.2 TB/s of
+// rows that miss the L2, which is what bounds them.
+template <int D, bool H, int U>
+__device__ inline void add_named_rows(const StepConfig& c, const RowNames<H>& names, uint32_t t0, uint32_t n, int lane,
+                                      float (&acc)[RowShape<D>::PL]) {
+  constexpr int PL = RowShape<D>::PL;
+  const uint32_t last = t0 + n - 1u;
+  if constexpr (H) {
+    constexpr int PW = (PL + 1) / 2;  // packed words per lane
+    uint32_t w[U][PW];
+    float sc[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t t = min(t0 + (uint32_t)u, last);
+      load_packed_f16<D>(c.adjh + (size_t)lane_value(names.slot, t) * D, lane, w[u]);
+      const float s = __uint_as_float(lane_value(__float_as_uint(names.scale), t));
+      sc[u] = (uint32_t)u < n ? s : 0.f;  // rows past n count as zero (FP16 rows are finite)
+    }
+    float r[U / 2][PL];
+#pragma unroll
+    for (int u = 0; u < U; u += 2)
+#pragma unroll
+      for (int q = 0; q < PL; ++q)
+        r[u / 2][q] = __builtin_fmaf(packed_half(w[u + 1], q), sc[u + 1], packed_half(w[u], q) * sc[u]);
+    add_rows_tree<U / 2, PL>(acc, r, (uint32_t)(U / 2));
+  } else {
+    float r[U][PL];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      load_slice<D>(c.adj + (size_t)lane_value(names.slot, min(t0 + (uint32_t)u, last)) * D, lane, r[u]);
+    add_rows_tree<U, PL>(acc, r, n);
+  }
+}
+
 // Partial sums of the pieces of long rows (each piece: <= kPieceEntries entries of one
 // run), by block blk of grid.
 template <int D, bool H>
@@ -2724,37 +2778,32 @@ __device__ inline void piece_sums(const StepConfig& c, StepState* st, const uint
   constexpr int PL = RowShape<D>::PL;
   constexpr int U = SR_UNROLL;
   const int lane = threadIdx.x & 63;
-  const uint32_t gw = blk * NW + (threadIdx.x >> 6);
+  const uint32_t wave = wave_uniform(threadIdx.x >> 6);
+  const uint32_t gw = blk * NW + wave;
   const uint32_t nwaves = grid * NW;
   const uint32_t np = st->n_pieces < c.piece_cap ? st->n_pieces : c.piece_cap;
-  // Batch by batch: a piece reads adjoint rows of its batch only, so every wave working
-  // on the same batch keeps the rows being read within one batch's share of the adjoint
-  // buffer (which the memory-side cache can hold) instead of all of them.
-  for (uint32_t bq = 0; bq <= c.pmask; ++bq)
-  for (uint32_t gp = gw; gp < np; gp += nwaves) {
-    const uint32_t info = c.piece_info[gp];
-    if ((info >> 29) != bq) continue;
-    const uint32_t s0 = c.piece_st[gp];
+  auto sum_piece = [&](uint32_t gp, uint32_t info) {
+    const uint32_t s0 = wave_uniform(c.piece_st[gp]);
     const uint32_t m = info & 0x1fffffffu;  // entries: a multiple of PIECE at most
     float acc[PL];
 #pragma unroll
     for (int q = 0; q < PL; ++q) acc[q] = 0.f;
     for (uint32_t c0 = 0; c0 < m; c0 += 64u) {  // 64 slots per lane-held chunk
       const uint32_t mm = m - c0 < 64u ? m - c0 : 64u;
-      const uint32_t sj = (uint32_t)lane < mm ? (Ss[s0 + c0 + lane] & kSlotMask) : 0u;
-      for (uint32_t t0 = 0; t0 < mm; t0 += U) {
-        float r[U][PL];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const uint32_t t = (t0 + u < mm) ? (t0 + u) : (mm - 1u);
-          const uint32_t s = __shfl(sj, (int)t, EP_WAVE);
-          load_adj_row<D, H>(c, s, lane, r[u]);
-        }
-        add_rows_tree<U, PL>(acc, r, mm - t0);
-      }
+      const RowNames<H> names =
+          row_names<H>(c, Ss[s0 + c0 + min((uint32_t)lane, mm - 1u)] & kSlotMask);
+      for (uint32_t t0 = 0; t0 < mm; t0 += U) add_named_rows<D, H, U>(c, names, t0, mm - t0, lane, acc);
     }
     store_slice<D>(c.part + (size_t)gp * D, lane, acc);
-  }
+  };
+  // Batch by batch: a piece reads adjoint rows of its batch only, so every wave working
+  // on the same batch keeps the rows being read within one batch's share of the adjoint
+  // buffer (which the memory-side cache can hold) instead of all of them.
+  for (uint32_t bq = 0; bq <= c.pmask; ++bq)
+    for (uint32_t gp = gw; gp < np; gp += nwaves) {
+      const uint32_t info = wave_uniform(c.piece_info[gp]);
+      if ((info >> 29) == bq) sum_piece(gp, info);
+    }
 }
 
 // The medium rows of the plan regions, dealt to the waves of grid blocks: one wave per row
@@ -2766,7 +2815,7 @@ __device__ inline void medium_rows(const StepConfig& c, StepState* st, const uin
   constexpr int U = SR_UNROLL;
   __shared__ float s_lr[kMaxGroup], s_sd[kMaxGroup];
   const int lane = threadIdx.x & 63;
-  const uint32_t gw = blk * NW + (threadIdx.x >> 6);
+  const uint32_t gw = blk * NW + wave_uniform(threadIdx.x >> 6);
   const uint32_t nwaves = grid * NW;
   if (threadIdx.x < kMaxGroup) {
     s_lr[threadIdx.x] = st->lr[threadIdx.x];
@@ -2784,13 +2833,13 @@ __device__ inline void medium_rows(const StepConfig& c, StepState* st, const uin
     const uint2* recs = c.mrec + (size_t)reg * cpr * 2u;
     for (uint32_t k = 0; k < nmed; ++k) {
       const uint2 rec = recs[k];
-      const uint32_t start = rec.x, len = rec.y;  // 32 < len <= 128
+      const uint32_t start = wave_uniform(rec.x), len = wave_uniform(rec.y);  // 32 < len <= 128
       const uint32_t e0 = (uint32_t)lane, e1 = 64u + (uint32_t)lane;
-      const uint32_t kk0 = e0 < len ? Ss[start + e0] >> kSlotBatchShift : 0u;  // batches
-      const uint32_t kk1 = e1 < len ? Ss[start + e1] >> kSlotBatchShift : 0u;
-      const uint32_t ss0 = e0 < len ? (Ss[start + e0] & kSlotMask) : 0u;
-      const uint32_t ss1 = e1 < len ? (Ss[start + e1] & kSlotMask) : 0u;
-      const uint32_t f = row_of_key(c, Ks[start]);
+      const uint32_t v0 = Ss[start + min(e0, len - 1u)], v1 = Ss[start + min(e1, len - 1u)];
+      const uint32_t kk0 = e0 < len ? v0 >> kSlotBatchShift : 0u;  // batches
+      const uint32_t kk1 = e1 < len ? v1 >> kSlotBatchShift : 0u;
+      const RowNames<H> names[2] = {row_names<H>(c, v0 & kSlotMask), row_names<H>(c, v1 & kSlotMask)};
+      const uint32_t f = wave_uniform(row_of_key(c, Ks[start]));
       float th[PL], mo[PL], va[PL];
       if (!c.grad_out) load_row_state<D>(c, f, lane, th, mo, va);
       const uint32_t last0 = __shfl(kk0, 63, EP_WAVE);
@@ -2805,22 +2854,24 @@ __device__ inline void medium_rows(const StepConfig& c, StepState* st, const uin
         if (rs0) rs0 &= rs0 - 1ull; else rs1 &= rs1 - 1ull;
         const uint32_t z = rs0 ? (uint32_t)(__ffsll((unsigned long long)rs0) - 1)
                                : (rs1 ? 64u + (uint32_t)(__ffsll((unsigned long long)rs1) - 1) : len);
-        const uint32_t ka = __shfl(kk0, (int)(a & 63u), EP_WAVE);
-        const uint32_t kb = __shfl(kk1, (int)(a & 63u), EP_WAVE);
-        const uint32_t bq = a < 64u ? ka : kb;
+        const uint32_t bq = a < 64u ? lane_value(kk0, a) : lane_value(kk1, a & 63u);
         float acc[PL];
   #pragma unroll
         for (int q = 0; q < PL; ++q) acc[q] = 0.f;
         for (uint32_t t0 = a; t0 < z; t0 += U) {
-          float r[U][PL];
-  #pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const uint32_t t = (t0 + u < z) ? (t0 + u) : (z - 1u);
-            const uint32_t sa = __shfl(ss0, (int)(t & 63u), EP_WAVE);
-            const uint32_t sb = __shfl(ss1, (int)(t & 63u), EP_WAVE);
-            load_adj_row<D, H>(c, t < 64u ? sa : sb, lane, r[u]);
+          // rounds count from the run's start and may straddle the two register halves
+          const uint32_t zr = min(z, t0 + (uint32_t)U);
+          if (zr <= 64u) {
+            add_named_rows<D, H, U>(c, names[0], t0, z - t0 < (uint32_t)U ? z - t0 : (uint32_t)U, lane, acc);
+          } else if (t0 >= 64u) {
+            add_named_rows<D, H, U>(c, names[1], t0 - 64u, z - t0, lane, acc);
+          } else {
+            const uint32_t src = (t0 + (uint32_t)lane) & 63u;  // the round's rows moved to lanes 0..
+            const bool low = t0 + (uint32_t)lane < 64u;
+            const uint32_t sa = __shfl(names[0].slot, (int)src, EP_WAVE), sb = __shfl(names[1].slot, (int)src, EP_WAVE);
+            const float ca = __shfl(names[0].scale, (int)src, EP_WAVE), cb = __shfl(names[1].scale, (int)src, EP_WAVE);
+            add_named_rows<D, H, U>(c, RowNames<H>{low ? sa : sb, low ? ca : cb}, 0u, z - t0, lane, acc);
           }
-          add_rows_tree<U, PL>(acc, r, z - t0);
         }
         upd |= apply_run<D>(c, st, sv, s_lr[bq], s_sd[bq], f, bq, lane, acc, th, mo, va);
       }
@@ -2866,7 +2917,7 @@ __global__ __launch_bounds__(256) void k_long_combine(StepConfig c, StepState* s
   // 4 waves per SIMD instead of 3 (its runs hold a few pieces each)
   constexpr int U = PL >= 4 ? 8 : SR_UNROLL;
   const int lane = threadIdx.x & 63;
-  const uint32_t gw = blockIdx.x * NW + (threadIdx.x >> 6);
+  const uint32_t gw = blockIdx.x * NW + wave_uniform(threadIdx.x >> 6);
   const uint32_t nwaves = gridDim.x * NW;
   const uint32_t nl = st->n_long < c.long_cap ? st->n_long : c.long_cap;
   const StepScalars sv = step_scalars(st);
@@ -2878,17 +2929,18 @@ __global__ __launch_bounds__(256) void k_long_combine(StepConfig c, StepState* s
   __syncthreads();
   uint32_t done = 0;
   for (uint32_t idx = gw; idx < nl; idx += nwaves) {
-    const uint32_t pb0 = c.long_pbase[idx];
-    const uint32_t nruns = c.long_len[idx];
-    const uint32_t f = row_of_key(c, Ks[c.long_st[idx]]);
+    const uint32_t pb0 = wave_uniform(c.long_pbase[idx]);
+    const uint32_t nruns = wave_uniform(c.long_len[idx]);
+    const uint32_t st0 = wave_uniform(c.long_st[idx]);
+    const uint32_t f = wave_uniform(row_of_key(c, Ks[st0]));
     float th[PL], m[PL], v[PL];
     if (!c.grad_out) load_row_state<D>(c, f, lane, th, m, v);
     bool upd = false;
     uint32_t pb = pb0;
-    uint32_t cur = c.long_st[idx];  // first entry of the current run
+    uint32_t cur = st0;  // first entry of the current run
     for (uint32_t jr = 0; jr < nruns && jr < kMaxGroup; ++jr) {
-      const uint32_t rinfo = c.long_runs[(size_t)idx * kMaxGroup + jr];
-      const uint32_t rlen = c.long_rlen[(size_t)idx * kMaxGroup + jr];
+      const uint32_t rinfo = wave_uniform(c.long_runs[(size_t)idx * kMaxGroup + jr]);
+      const uint32_t rlen = wave_uniform(c.long_rlen[(size_t)idx * kMaxGroup + jr]);
       const uint32_t bq = (rinfo >> 24) & 7u;
       uint32_t pcs = rinfo & 0xffffffu;
       if (pb >= c.piece_cap) pcs = 0u;
@@ -2898,16 +2950,8 @@ __global__ __launch_bounds__(256) void k_long_combine(StepConfig c, StepState* s
       for (int q = 0; q < PL; ++q) acc[q] = 0.f;
       if ((rinfo & 0xffffffu) == 0u) {
         // a run of at most PIECE entries: its adjoint rows in entry order
-        const uint32_t sj = (uint32_t)lane < rlen ? (Ss[cur + lane] & kSlotMask) : 0u;
-        for (uint32_t t0 = 0; t0 < rlen; t0 += U) {
-          float r[U][PL];
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const uint32_t t = (t0 + u < rlen) ? (t0 + u) : (rlen - 1u);
-            load_adj_row<D, H>(c, __shfl(sj, (int)t, EP_WAVE), lane, r[u]);
-          }
-          add_rows_tree<U, PL>(acc, r, rlen - t0);
-        }
+        const RowNames<H> names = row_names<H>(c, Ss[cur + min((uint32_t)lane, rlen - 1u)] & kSlotMask);
+        for (uint32_t t0 = 0; t0 < rlen; t0 += U) add_named_rows<D, H, U>(c, names, t0, rlen - t0, lane, acc);
       }
       for (uint32_t j0 = 0; j0 < pcs; j0 += U) {
         float r[U][PL];
