@@ -4,11 +4,13 @@
 
 #include <algorithm>
 #include <cmath>
+#include <condition_variable>
 #include <cstdio>
 #include <cstring>
 #include <iterator>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <type_traits>
 #include <vector>
 
@@ -57,6 +59,141 @@ void shuffle(std::vector<T>& v, HostRng& r) {
   for (size_t i = v.size(); i > 1; --i) std::swap(v[i - 1], v[r.below(i)]);
 }
 
+// Copies device memory to a caller's (pageable) array after the work queued on the stream.  From
+// kMinBytes up through a ring of pinned chunks: the copy engine fills chunks while a few
+// threads move filled ones out, taking the page faults of a fresh array side by side.  The
+// runtime's own pageable copy waits for the faults and the transfer in turn: 51 MB into a fresh
+// array take it 5.2 ms on a MI355X host and 3.0 into a touched one, the transfer alone 1.0;
+// this takes 1.6.  The ring (8 MB) belongs to one context or aligner, from its first large
+// copy to its end; the threads end with the copy.
+class HostCopy {
+ public:
+  HostCopy() = default;
+  HostCopy(const HostCopy&) = delete;
+  HostCopy& operator=(const HostCopy&) = delete;
+  ~HostCopy() {
+    for (hipEvent_t e : ev_)
+      if (e) (void)hipEventDestroy(e);
+    if (ring_) (void)hipHostFree(ring_);
+  }
+
+  hipError_t run(void* dst, const void* src, size_t bytes, hipStream_t s) {
+    if (bytes >= kMinBytes && prepare() && start()) return copy((unsigned char*)dst, (const unsigned char*)src, bytes, s);
+    hipError_t e = bytes ? hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s) : hipSuccess;
+    return e == hipSuccess ? hipStreamSynchronize(s) : e;
+  }
+
+ private:
+  static constexpr size_t kMinBytes = (size_t)8 << 20, kChunk = (size_t)1 << 20;
+  static constexpr int kRing = 8, kFlight = 3, kThreads = 6;  // chunks, copies in flight, threads
+
+  // The ring and its events; false when they are not to be had.
+  bool prepare() {
+    if (!ring_ && hipHostMalloc((void**)&ring_, kRing * kChunk, hipHostMallocDefault) != hipSuccess) {
+      ring_ = nullptr;
+      (void)hipGetLastError();
+      return false;
+    }
+    for (hipEvent_t& e : ev_)
+      if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+        e = nullptr;
+        (void)hipGetLastError();
+        return false;
+      }
+    return true;
+  }
+
+  // The threads of a copy: as many as there are to be had, false for none.
+  bool start() {
+    ready_ = taken_ = 0;
+    last_ = false;
+    for (size_t& n : out_) n = 0;
+    try {
+      for (std::thread& t : threads_) t = std::thread([this] { work(); });
+    } catch (...) {
+    }
+    return threads_[0].joinable();
+  }
+
+  hipError_t copy(unsigned char* dst, const unsigned char* src, size_t bytes, hipStream_t s) {
+    dst_ = dst;
+    bytes_ = bytes;
+    const size_t n = (bytes + kChunk - 1) / kChunk;
+    hipError_t e = hipSuccess;
+    for (size_t c = 0; c < n + kFlight && e == hipSuccess; ++c) {
+      if (c < n) {
+        if (c >= (size_t)kRing) {  // the chunk that used this part of the ring has left it
+          std::unique_lock<std::mutex> lk(mu_);
+          cv_.wait(lk, [&] { return out_[c % kRing] > (c - kRing) / kRing; });
+        }
+        e = hipMemcpyAsync(ring_ + c % kRing * kChunk, src + c * kChunk, std::min(kChunk, bytes - c * kChunk),
+                           hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipEventRecord(ev_[c % kRing], s);
+      }
+      if (e == hipSuccess && c >= (size_t)kFlight) {
+        e = hipEventSynchronize(ev_[(c - kFlight) % kRing]);
+        if (e == hipSuccess) {
+          std::lock_guard<std::mutex> lk(mu_);
+          ready_ = c - kFlight + 1;
+        }
+        cv_.notify_all();
+      }
+    }
+    if (e != hipSuccess) (void)hipStreamSynchronize(s);  // no copy into the ring may be left
+    stop(e != hipSuccess);
+    return e;
+  }
+
+  // The threads end: when every ready chunk has been moved out, or at once.
+  void stop(bool now) {
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      last_ = true;
+      if (now) taken_ = ready_;
+    }
+    cv_.notify_all();
+    for (std::thread& t : threads_)
+      if (t.joinable()) t.join();
+  }
+
+  void work() {
+    std::unique_lock<std::mutex> lk(mu_);
+    for (;;) {
+      cv_.wait(lk, [&] { return taken_ < ready_ || last_; });
+      if (taken_ >= ready_) return;
+      const size_t c = taken_++;
+      lk.unlock();
+      std::memcpy(dst_ + c * kChunk, ring_ + c % kRing * kChunk, std::min(kChunk, bytes_ - c * kChunk));
+      lk.lock();
+      ++out_[c % kRing];
+      cv_.notify_all();
+    }
+  }
+
+  unsigned char* ring_ = nullptr;
+  hipEvent_t ev_[kRing] = {};
+  std::thread threads_[kThreads];
+  std::mutex mu_;
+  std::condition_variable cv_;
+  unsigned char* dst_ = nullptr;
+  size_t bytes_ = 0;
+  size_t ready_ = 0, taken_ = 0;  // chunks filled, chunks given to a thread
+  size_t out_[kRing] = {};        // chunks moved out of each part of the ring
+  bool last_ = false;             // no more chunks will come
+};
+
+// Whether every one of n ids is below the limit (checked a block at a time, so that the
+// compare loop vectorises).
+bool ids_below(const uint32_t* ids, uint64_t n, uint32_t limit) {
+  for (uint64_t i = 0; i < n; i += 4096) {
+    const uint64_t e = std::min(n, i + 4096);
+    uint32_t bad = 0;
+    for (uint64_t j = i; j < e; ++j) bad |= ids[j] >= limit ? 1u : 0u;
+    if (bad) return false;
+  }
+  return true;
+}
+
 uint32_t next_pow2(uint64_t x) {
   uint64_t p = 1;
   while (p < x) p <<= 1;
@@ -76,6 +213,7 @@ struct ep_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   std::vector<void*> allocs;
+  HostCopy to_host;  // large results on their way to the caller
   unsigned char* scratch = nullptr;  // this device's `scratch` (device address)
 
   // graph / features
@@ -641,11 +779,12 @@ int upload_split(ep_ctx* c) {
   return EP_OK;
 }
 
-// Shuffle the train ids for a pass (mod.rs:173) and stage them to the device.
-int upload_pass_perm(ep_ctx* c, HostRng& rng) {
+// Stage the train ids, shuffled for a pass (mod.rs:173; here unless the caller has already),
+// to the device.
+int upload_pass_perm(ep_ctx* c, HostRng& rng, bool shuffled = false) {
   EP_HIP(hipStreamSynchronize(c->stream));
   std::vector<uint32_t>& t = c->train;
-  shuffle(t, rng);
+  if (!shuffled) shuffle(t, rng);
   std::memcpy(c->h_perm, t.data(), t.size() * sizeof(uint32_t));
   if (!t.empty())
     EP_HIP(hipMemcpyAsync(c->d_perm, c->h_perm, t.size() * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
@@ -1052,8 +1191,7 @@ static int copy_staged(ep_ctx* c, float* out, uint64_t rows, uint32_t D, bool* s
   for (uint64_t r = 0; r < rows && e == hipSuccess; r += chunk) {
     const uint64_t n = std::min(chunk, rows - r);
     e = stage(r, n, buf);
-    if (e == hipSuccess) e = hipMemcpyAsync(out + r * D, buf, n * row_bytes, hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess) e = c->to_host.run(out + r * D, buf, n * row_bytes, c->stream);
   }
   (void)hipFree(buf);
   if (e != hipSuccess) return fail(EP_EHIP, std::string("staged copy: ") + hipGetErrorString(e));
@@ -1102,7 +1240,7 @@ int ep_get_table(ep_ctx* c, float* rows) {
       std::memcpy(rows + i, &u, sizeof(float));
     }
   } else {
-    EP_HIP(hipMemcpy(rows, c->d_table, n * sizeof(float), hipMemcpyDeviceToHost));
+    EP_HIP(c->to_host.run(rows, c->d_table, n * sizeof(float), c->stream));
   }
   return EP_OK;
 }
@@ -1112,7 +1250,7 @@ int ep_get_table_bf16(ep_ctx* c, uint16_t* rows) {
   if (!c->table_ready || c->cfg.precision == EP_PREC_FP32) return fail(EP_ESTATE, "no bf16 table");
   EP_HIP(hipSetDevice(c->device));
   EP_HIP(hipStreamSynchronize(c->stream));
-  EP_HIP(hipMemcpy(rows, c->d_table, (size_t)c->n_vocab * row_width(c->cfg) * sizeof(uint16_t), hipMemcpyDeviceToHost));
+  EP_HIP(c->to_host.run(rows, c->d_table, (size_t)c->n_vocab * row_width(c->cfg) * sizeof(uint16_t), c->stream));
   return EP_OK;
 }
 
@@ -1176,9 +1314,10 @@ int ep_learn(ep_ctx* c, ep_progress_fn progress, void* user) {
   vc.steps_per_pass = (uint32_t)((c->valid.size() + vc.batch - 1) / vc.batch);
   vc.total_updates = 1;
   for (uint32_t pass = 1; pass <= c->cfg.passes; ++pass) {
-    EP_TRY(upload_pass_perm(c, rng));
+    EP_TRY(upload_pass_perm(c, rng, pass > 1));
     EP_TRY(set_pass(c, c->d_state, pass, pass == 1 ? &next_step : nullptr));
     for (uint32_t s = 0; s < spp; ++s) EP_TRY(run_step(c, sc));
+    if (pass < c->cfg.passes) shuffle(c->train, rng);  // the next pass's, while the device runs this one's steps
     EP_TRY(check_state_err(c));
     EP_HIP(hipMemcpy(losses.data(), c->d_pass_loss, losses.size() * sizeof(float), hipMemcpyDeviceToHost));
     // per-batch error = sum of contributing losses / batch size; pass error = mean over batches
@@ -1597,31 +1736,46 @@ int ep_bench_steps(ep_ctx* c, uint32_t warmup, uint32_t steps, int instrument, e
   return EP_OK;
 }
 
+// Inference over host feature lists: the lists, `extra` FP32 values and the output rows share
+// one device allocation; launch(lists, ids, extra, out) runs the aggregate on the context's
+// stream.  out[n_nodes * width] is copied back.
+extern "C++" template <typename Launch>
+static int embed_lists(ep_ctx* c, uint64_t n_nodes, const uint64_t* f_indptr, const uint32_t* f_ids, const float* extra,
+                       size_t n_extra, size_t width, float* out, Launch launch) {
+  EP_HIP(hipSetDevice(c->device));
+  const uint64_t tot = f_indptr[n_nodes];
+  const size_t out_bytes = (size_t)n_nodes * width * sizeof(float);
+  const size_t parts[] = {out_bytes, (n_nodes + 1) * sizeof(uint64_t), tot * sizeof(uint32_t), n_extra * sizeof(float)};
+  size_t at[4], total = 0;
+  for (int i = 0; i < 4; ++i) {
+    at[i] = total;
+    total += (std::max<size_t>(parts[i], 16) + 255) & ~(size_t)255;
+  }
+  unsigned char* buf = nullptr;
+  EP_TRY(c->alloc(&buf, total));
+  uint64_t* dp = (uint64_t*)(buf + at[1]);
+  uint32_t* di = (uint32_t*)(buf + at[2]);
+  float* dx = (float*)(buf + at[3]);
+  EP_HIP(hipMemcpy(dp, f_indptr, parts[1], hipMemcpyHostToDevice));
+  if (tot) EP_HIP(hipMemcpy(di, f_ids, parts[2], hipMemcpyHostToDevice));
+  if (n_extra) EP_HIP(hipMemcpy(dx, extra, parts[3], hipMemcpyHostToDevice));
+  refresh_base(c);
+  EP_HIP(launch(dp, di, dx, (float*)(buf + at[0])));
+  EP_HIP(c->to_host.run(out, buf + at[0], out_bytes, c->stream));
+  c->release(buf);
+  return EP_OK;
+}
+
 int ep_embed_averaged(ep_ctx* c, uint64_t n_nodes, const uint64_t* f_indptr, const uint32_t* f_ids, float* out) {
   if (!c || !f_indptr || !out) return fail(EP_EINVAL, "NULL argument");
   if (!c->table_ready) return fail(EP_ESTATE, "no table");
-  const uint64_t tot = f_indptr[n_nodes];
   for (uint64_t i = 0; i < n_nodes; ++i)
     if (f_indptr[i + 1] < f_indptr[i]) return fail(EP_EINVAL, "f_indptr must be non-decreasing");
-  for (uint64_t i = 0; i < tot; ++i)
-    if (f_ids[i] >= c->n_vocab) return fail(EP_EINVAL, "feature id out of range");
-  EP_HIP(hipSetDevice(c->device));
-  uint64_t* dp = nullptr;
-  uint32_t* di = nullptr;
-  float* dout = nullptr;
-  EP_TRY(c->alloc(&dp, n_nodes + 1));
-  EP_TRY(c->alloc(&di, tot));
-  EP_TRY(c->alloc(&dout, (size_t)n_nodes * row_width(c->cfg)));
-  EP_HIP(hipMemcpy(dp, f_indptr, (n_nodes + 1) * sizeof(uint64_t), hipMemcpyHostToDevice));
-  if (tot) EP_HIP(hipMemcpy(di, f_ids, tot * sizeof(uint32_t), hipMemcpyHostToDevice));
-  refresh_base(c);
-  EP_HIP(ep::launch_embed_averaged(c->base, dp, di, n_nodes, dout, c->stream));
-  EP_HIP(hipStreamSynchronize(c->stream));
-  EP_HIP(hipMemcpy(out, dout, (size_t)n_nodes * row_width(c->cfg) * sizeof(float), hipMemcpyDeviceToHost));
-  c->release(dp);
-  c->release(di);
-  c->release(dout);
-  return EP_OK;
+  if (!ids_below(f_ids, f_indptr[n_nodes], c->n_vocab)) return fail(EP_EINVAL, "feature id out of range");
+  return embed_lists(c, n_nodes, f_indptr, f_ids, nullptr, 0, row_width(c->cfg), out,
+                     [&](const uint64_t* dp, const uint32_t* di, const float*, float* dout) {
+                       return ep::launch_embed_averaged(c->base, dp, di, n_nodes, dout, c->stream);
+                     });
 }
 
 int ep_embed_weighted(ep_ctx* c, uint64_t n_nodes, const uint64_t* f_indptr, const uint32_t* f_ids,
@@ -1629,66 +1783,30 @@ int ep_embed_weighted(ep_ctx* c, uint64_t n_nodes, const uint64_t* f_indptr, con
   if (!c || !f_indptr || !out || !p_w) return fail(EP_EINVAL, "NULL argument");
   if (!c->table_ready) return fail(EP_ESTATE, "no table");
   if (!(alpha > 0.f) || !std::isfinite(alpha)) return fail(EP_EINVAL, "alpha must be finite and > 0");
-  const uint64_t tot = f_indptr[n_nodes];
   for (uint64_t i = 0; i < n_nodes; ++i)
     if (f_indptr[i + 1] < f_indptr[i]) return fail(EP_EINVAL, "f_indptr must be non-decreasing");
-  for (uint64_t i = 0; i < tot; ++i)
-    if (f_ids[i] >= c->n_vocab || f_ids[i] >= n_p) return fail(EP_EINVAL, "feature id out of range");
+  if (!ids_below(f_ids, f_indptr[n_nodes], std::min(c->n_vocab, n_p))) return fail(EP_EINVAL, "feature id out of range");
   for (uint32_t i = 0; i < n_p; ++i)
     if (!(p_w[i] >= 0.f)) return fail(EP_EINVAL, "unigram probabilities must be >= 0");
-  EP_HIP(hipSetDevice(c->device));
-  const size_t W = row_width(c->cfg);
-  uint64_t* dp = nullptr;
-  uint32_t* di = nullptr;
-  float* dw = nullptr;
-  float* dout = nullptr;
-  EP_TRY(c->alloc(&dp, n_nodes + 1));
-  EP_TRY(c->alloc(&di, tot));
-  EP_TRY(c->alloc(&dw, n_p));
-  EP_TRY(c->alloc(&dout, (size_t)n_nodes * W));
-  EP_HIP(hipMemcpy(dp, f_indptr, (n_nodes + 1) * sizeof(uint64_t), hipMemcpyHostToDevice));
-  if (tot) EP_HIP(hipMemcpy(di, f_ids, tot * sizeof(uint32_t), hipMemcpyHostToDevice));
-  EP_HIP(hipMemcpy(dw, p_w, (size_t)n_p * sizeof(float), hipMemcpyHostToDevice));
-  refresh_base(c);
-  EP_HIP(ep::launch_embed_weighted(c->base, dp, di, dw, alpha, n_nodes, dout, c->stream));
-  EP_HIP(hipStreamSynchronize(c->stream));
-  EP_HIP(hipMemcpy(out, dout, (size_t)n_nodes * W * sizeof(float), hipMemcpyDeviceToHost));
-  c->release(dp);
-  c->release(di);
-  c->release(dw);
-  c->release(dout);
-  return EP_OK;
+  return embed_lists(c, n_nodes, f_indptr, f_ids, p_w, n_p, row_width(c->cfg), out,
+                     [&](const uint64_t* dp, const uint32_t* di, const float* dw, float* dout) {
+                       return ep::launch_embed_weighted(c->base, dp, di, dw, alpha, n_nodes, dout, c->stream);
+                     });
 }
 
 int ep_embed_attention(ep_ctx* c, uint64_t n_nodes, const uint64_t* f_indptr, const uint32_t* f_ids, float* out) {
   if (!c || !f_indptr || !out) return fail(EP_EINVAL, "NULL argument");
   if (!c->table_ready) return fail(EP_ESTATE, "no table");
   if (c->cfg.attention_dk == 0) return fail(EP_ESTATE, "the context is not configured for attention");
-  const uint64_t tot = f_indptr[n_nodes];
   for (uint64_t i = 0; i < n_nodes; ++i) {
     if (f_indptr[i + 1] < f_indptr[i]) return fail(EP_EINVAL, "f_indptr must be non-decreasing");
     if (f_indptr[i + 1] - f_indptr[i] > 64) return fail(EP_EINVAL, "attention supports at most 64 features per node");
   }
-  for (uint64_t i = 0; i < tot; ++i)
-    if (f_ids[i] >= c->n_vocab) return fail(EP_EINVAL, "feature id out of range");
-  EP_HIP(hipSetDevice(c->device));
-  const size_t dm = c->cfg.dims;
-  uint64_t* dp = nullptr;
-  uint32_t* di = nullptr;
-  float* dout = nullptr;
-  EP_TRY(c->alloc(&dp, n_nodes + 1));
-  EP_TRY(c->alloc(&di, tot));
-  EP_TRY(c->alloc(&dout, (size_t)n_nodes * dm));
-  EP_HIP(hipMemcpy(dp, f_indptr, (n_nodes + 1) * sizeof(uint64_t), hipMemcpyHostToDevice));
-  if (tot) EP_HIP(hipMemcpy(di, f_ids, tot * sizeof(uint32_t), hipMemcpyHostToDevice));
-  refresh_base(c);
-  EP_HIP(ep::launch_att_embed(c->base, dp, di, n_nodes, dout, c->stream));
-  EP_HIP(hipStreamSynchronize(c->stream));
-  EP_HIP(hipMemcpy(out, dout, (size_t)n_nodes * dm * sizeof(float), hipMemcpyDeviceToHost));
-  c->release(dp);
-  c->release(di);
-  c->release(dout);
-  return EP_OK;
+  if (!ids_below(f_ids, f_indptr[n_nodes], c->n_vocab)) return fail(EP_EINVAL, "feature id out of range");
+  return embed_lists(c, n_nodes, f_indptr, f_ids, nullptr, 0, c->cfg.dims, out,
+                     [&](const uint64_t* dp, const uint32_t* di, const float*, float* dout) {
+                       return ep::launch_att_embed(c->base, dp, di, n_nodes, dout, c->stream);
+                     });
 }
 
 // NeighborhoodAligner (alignment.rs, lib.rs:3040-3171): the graph (with its edge CDF) and
@@ -1704,6 +1822,7 @@ struct ep_aligner {
   float* emb = nullptr;
   float* out = nullptr;
   uint64_t out_rows = 0;
+  HostCopy to_host;
   hipEvent_t ev[2] = {nullptr, nullptr};
   float last_ms = 0.f;  // duration of the last run's kernel (HIP events)
 };
@@ -1775,8 +1894,7 @@ int ep_aligner_run(ep_aligner* a, float alpha, uint32_t max_neighbors, uint64_t 
   EP_HIP(ep::launch_align((int)a->dims, a->emb, a->indptr, a->indices, a->cdf, adaptive ? 0.f : alpha, adaptive,
                           max_neighbors, first, count, a->out, a->stream));
   EP_HIP(hipEventRecord(a->ev[1], a->stream));
-  EP_HIP(hipMemcpyAsync(out, a->out, (size_t)count * a->dims * sizeof(float), hipMemcpyDeviceToHost, a->stream));
-  EP_HIP(hipStreamSynchronize(a->stream));
+  EP_HIP(a->to_host.run(out, a->out, (size_t)count * a->dims * sizeof(float), a->stream));
   EP_HIP(hipEventElapsedTime(&a->last_ms, a->ev[0], a->ev[1]));
   return EP_OK;
 }

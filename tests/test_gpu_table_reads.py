@@ -54,3 +54,51 @@ def test_moments_after_a_step(prec):
     # one FP32 product for m, two for v: 2 and 3 roundings of 2^-24
     assert np.all(np.abs(m - b1.astype(np.float64) * g) <= 2 * 2.0**-24 * np.abs(m))
     assert np.all(np.abs(v - b2.astype(np.float64) * g.astype(np.float64) ** 2) <= 3 * 2.0**-24 * np.abs(v) + 1e-44)
+
+
+def test_large_reads_from_two_threads():
+    """Copies of 8 MiB and more go through a pinned ring and helper threads of their own."""
+    import threading
+
+    tables = [np.random.default_rng(k).standard_normal((150_001 + k, 64)).astype(np.float32) for k in range(2)]
+    got = [[], []]
+
+    def work(k):
+        cfg = N.default_config()
+        cfg.dims = 64
+        with N.Context(cfg) as ctx:
+            ctx.set_features(np.array([0, 1], np.uint64), np.array([0], np.uint32), len(tables[k]))
+            ctx.set_table(tables[k])
+            got[k] = [np.array_equal(ctx.get_table(), tables[k]) for _ in range(5)]
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert got == [[True] * 5] * 2
+
+
+@pytest.mark.parametrize("nodes", [32_767, 32_768, 40_000])  # either side of 8 MiB of output rows
+def test_embedding_large_node_sets(nodes):
+    rng = np.random.default_rng(nodes)
+    table = rng.standard_normal((500, 64)).astype(np.float32)
+    counts = rng.integers(0, 4, size=nodes)
+    ip = np.concatenate([[0], np.cumsum(counts)]).astype(np.uint64)
+    ids = rng.integers(0, 500, size=int(ip[-1])).astype(np.uint32)
+    cfg = N.default_config()
+    cfg.dims = 64
+    with N.Context(cfg) as ctx:
+        ctx.set_features(np.array([0, 1], np.uint64), np.array([0], np.uint32), 500)
+        ctx.set_table(table)
+        out = ctx.embed_averaged(ip, ids)
+        for bad in (0, 4095, 4096, len(ids) - 1):  # the id check's blocks of 4096
+            wrong = ids.copy()
+            wrong[bad] = 500
+            with pytest.raises(N.NativeError, match="feature id out of range"):
+                ctx.embed_averaged(ip, wrong)
+    want = np.zeros((nodes, 64))
+    np.add.at(want, np.repeat(np.arange(nodes), counts), table[ids].astype(np.float64))
+    want[counts > 0] /= counts[counts > 0, None]
+    # at most 3 rows added and one division: 3 roundings of 2^-24 of sums below 3 max |row|
+    assert np.max(np.abs(out - want)) <= 4 * 3 * 2.0**-24 * np.abs(table).max()
