@@ -24,8 +24,8 @@
 // 8 (r / 4) + 4 (l / 32) + r % 4 of its registers r.  Two layouts of the scores:
 //   K Q^T  (lane = query i, registers = keys j): the row softmax needs only the partner
 //          lane l ^ 32; the probabilities there are the A operand of dQ = dT K;
-//   Q K^T  (lane = key j, registers = queries i): column sums w_j need only the
-//          partner lane; the probabilities there are the A operand of dK = dT^T Q.
+//   its transpose (lane = key j, registers = queries i; turned over through the LDS): column
+//          sums w_j need only the partner lane; the A operand of dK = dT^T Q.
 //
 // k_att_forward   block outputs
 // k_att_loss      one wave per example: a, p = mean of the neighbour blocks, n_k; margin
@@ -143,8 +143,6 @@ __device__ inline void ld8<uint16_t>(const uint16_t* p, float (&v)[8]) {
 // LDS of one block's wave (floats / words).  The per-item arrays come first; the last
 // region holds the Q / K operand tiles (backward) or the value accumulators (forward).
 struct AttLds {
-  float* M;      // [64] row max of the scaled scores
-  float* iZ;     // [64] 1 / softmax denominator
   float* r;      // [64] sum_j A_ij u_j
   uint32_t* f;   // [64] feature of each item
   float* cnt;    // [64] count of each item
@@ -229,16 +227,17 @@ constexpr int kMaxHeads = 16;
 
 // Per-item arrays.  Random attention adds the 64 row masks in front; the backward works
 // one head at a time and keeps u for that head only (no w).  LDS per block bounds the
-// blocks per CU of the backward: at H = 4, d = 128 it takes 19968 bytes, 8 blocks per CU
-// (the VGPR bound), where 20992 would allow 7.
+// blocks per CU of the backward: at H = 4, d = 128 it takes 19456 bytes, 8 blocks per CU
+// (the VGPR bound), where 20481 would allow 7.
 __host__ __device__ inline size_t att_lds_small(int dm, int H, bool rnd, bool backward) {
-  return (rnd ? 2 * (size_t)kAttMaxItems : 0) + 7 * (size_t)kAttMaxItems +
+  return (rnd ? 2 * (size_t)kAttMaxItems : 0) + 5 * (size_t)kAttMaxItems +
          (backward ? (size_t)kAttMaxItems : 2 * (size_t)kAttMaxItems * H) + (size_t)((dm + 3) & ~3);
 }
 
-// forward: the value accumulators; backward: the operand tiles
+// forward: a tile being turned over, then the value accumulators; backward: the operand tiles
 __host__ __device__ inline size_t att_lds_floats(int dm, int H, bool backward, bool rnd) {
-  return att_lds_small(dm, H, rnd, backward) + (backward ? 2 * (size_t)kAttMaxItems * kTileStride : (size_t)H * dm);
+  const size_t vals = (size_t)H * dm, tile = 32 * (size_t)kTileStride;
+  return att_lds_small(dm, H, rnd, backward) + (backward ? 4 * tile : vals > tile ? vals : tile);
 }
 
 __device__ inline AttLds att_lds(float* sm, int dm, int H, uint32_t win, bool rnd, bool backward = false) {
@@ -249,9 +248,7 @@ __device__ inline AttLds att_lds(float* sm, int dm, int H, uint32_t win, bool rn
   L.rk = 0u;
   L.rp = 0.f;
   L.rpos = L.rpass = L.re = L.k0 = L.k1 = 0u;
-  L.M = sm + (rnd ? 2 * kAttMaxItems : 0);  // after the 64 row masks (Random attention)
-  L.iZ = L.M + kAttMaxItems;
-  L.r = L.iZ + kAttMaxItems;
+  L.r = sm + (rnd ? 2 * kAttMaxItems : 0);  // after the 64 row masks (Random attention)
   L.f = (uint32_t*)(L.r + kAttMaxItems);
   L.cnt = (float*)(L.f + kAttMaxItems);
   L.q = (uint32_t*)(L.cnt + kAttMaxItems);
@@ -440,10 +437,11 @@ __device__ inline f32x16 score_tile(const QKop<uint16_t>& a, const QKop<uint16_t
 }
 
 // Row statistics of query tile I from the K Q^T tiles: scaled, masked scores into T,
-// returns the row max and 1 / denominator of query i = 32 I + l % 32 (both halves).
+// turned into exp(score - row max); returns 1 / denominator of query i = 32 I + l % 32 (both
+// halves).
 template <int AM>
 __device__ inline void row_softmax_stats(f32x16 (&T)[2], int NT, uint32_t n, int I, float ci, const AttLds& L,
-                                         float isq, float* mx_out, float* iz_out) {
+                                         float isq, float* iz_out) {
   const int l = (int)lane_id();
   const uint32_t i = 32u * I + (l & 31);
   float mx = -INFINITY;
@@ -473,8 +471,31 @@ __device__ inline void row_softmax_stats(f32x16 (&T)[2], int NT, uint32_t n, int
     }
   }
   z += __shfl_xor(z, 32, EP_WAVE);
-  *mx_out = m0;
   *iz_out = (i < n) ? 1.0f / z : 0.f;
+}
+
+// A 32 x 32 tile turned over through the LDS, so that lanes and registers swap roles: from
+// lane = query i, registers = keys j (row_softmax_stats) to lane = key j, registers =
+// queries i.  buf holds 32 rows of kTileStride floats; the block is the wave, so the barrier
+// between the two is its own wait.  Computing the second form on the matrix cores again took
+// 16 FP32 instructions (1024 cycles) and 16 exponentials per tile; this takes 16 LDS writes
+// and 8 paired reads, and the values are the same bits.
+__device__ inline void put_tile(float* buf, const f32x16& T) {
+  const int l = (int)lane_id();
+#pragma unroll
+  for (int r = 0; r < 16; ++r) buf[mrow(r, l) * kTileStride + (l & 31)] = T[r];
+}
+__device__ inline f32x16 get_tile_turned(const float* buf) {
+  const int l = (int)lane_id();
+  const float* row = buf + (l & 31) * kTileStride + 4 * (l >> 5);
+  f32x16 T;
+#pragma unroll
+  for (int r = 0; r < 16; r += 2) {
+    const float2 x = *reinterpret_cast<const float2*>(row + 8 * (r >> 2) + (r & 3));
+    T[r] = x.x;
+    T[r + 1] = x.y;
+  }
+  return T;
 }
 
 }  // namespace
@@ -552,7 +573,9 @@ __device__ inline void att_block_output(const T* __restrict__ table, uint32_t W,
       const bool ok = I < NT && i < n;
       load_qk<DK, T>(table + (size_t)(ok ? L.f[i] : 0u) * W, ok, h, H, hf, qa[I], ka[I]);
     }
-    // softmax statistics per query row from the K Q^T tiles
+    // per query tile: scores (K Q^T) and softmax; each tile of probabilities turned over adds
+    // to the column sums w_jh of its keys (one per lane)
+    float wj[2] = {0.f, 0.f};
 #pragma unroll
     for (int I = 0; I < 2; ++I) {
       if (I >= NT) break;
@@ -564,33 +587,29 @@ __device__ inline void att_block_output(const T* __restrict__ table, uint32_t W,
       }
       const uint32_t i = 32u * I + c32;
       const float ci = i < n ? L.cnt[i] : 0.f;
-      float mx, iz;
-      row_softmax_stats<AM>(Tt, NT, n, I, ci, L, isq_h, &mx, &iz);
-      if (hf == 0) { L.M[i] = mx; L.iZ[i] = iz; }
+      float iz;
+      row_softmax_stats<AM>(Tt, NT, n, I, ci, L, isq_h, &iz);
+#pragma unroll
+      for (int J = 0; J < 2; ++J) {
+        if (J >= NT) break;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) Tt[J][r] = i < n ? Tt[J][r] * iz : 0.f;  // padded queries: no part
+        put_tile(L.acc, Tt[J]);
+        __syncthreads();
+        const f32x16 A = get_tile_turned(L.acc);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) wj[J] += A[r];
+        __syncthreads();
+      }
     }
-    __syncthreads();
-    // column sums w_jh from the Q K^T tiles
 #pragma unroll
     for (int J = 0; J < 2; ++J) {
       if (J >= NT) break;
       const uint32_t j = 32u * J + c32;
-      const float cj = j < n ? L.cnt[j] : 0.f;
-      float wj = 0.f;
-#pragma unroll
-      for (int I = 0; I < 2; ++I) {
-        if (I >= NT) break;
-        const f32x16 a = score_tile<DK>(qa[I], ka[J], f32x16{});
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const uint32_t i = 32u * I + mrow(r, l);
-          const float sc = a[r] * count_factor(L.cnt[i], cj) * isq_h;
-          wj += att_pair<AM>(L, i, j, n) ? softmax_exp(sc - L.M[i]) * L.iZ[i] : 0.f;
-        }
-      }
-      wj += __shfl_xor(wj, 32, EP_WAVE);
-      if (hf == 0) L.w[j * H + h] = j < n ? wj * hs : 0.f;
+      const float w = wj[J] + __shfl_xor(wj[J], 32, EP_WAVE);
+      if (hf == 0) L.w[j * H + h] = j < n ? w * hs : 0.f;
     }
-    __syncthreads();  // the next head rewrites the row statistics read above
+    __syncthreads();
   }
   // value sweep: lane l covers 8 consecutive values p of an item's value part
   const int VP = H * dm;
@@ -648,10 +667,14 @@ __device__ inline void att_random_setup(const StepConfig& c, const StepState* st
 }
 
 // ------------------------------------------------------------------------------------
-// k_att_forward: one wave (64-thread block) per attention block.
+// k_att_forward: one wave (64-thread block) per attention block.  Four waves per SIMD asked
+// for: the compiler then keeps the matrix results out of accumulation registers (122 VGPRs
+// in all, no spills; 143 without; Sliding and Random would spill and are left to it).  31.7k blocks of 32 items on average, 4 heads, d_k 32, d 128, FP32:
+// 560 -> 348 us with one matrix product per tile pair instead of two (see put_tile); what is
+// left is the latency of the row loads and the softmax of the padded tiles.
 // ------------------------------------------------------------------------------------
 template <int DK, typename T, int AM>
-__global__ __launch_bounds__(64) void k_att_forward(StepConfig c, StepState* st) {
+__global__ __launch_bounds__(64, AM == AM_FULL ? 4 : 1) void k_att_forward(StepConfig c, StepState* st) {
   extern __shared__ float sm[];
   const int H = c.att_heads, dm = c.att_dm;
   AttLds L = att_lds(sm, dm, H, c.att_win, AM == AM_RANDOM);
@@ -666,10 +689,11 @@ __global__ __launch_bounds__(64) void k_att_forward(StepConfig c, StepState* st)
 // ------------------------------------------------------------------------------------
 // k_att_embed: AttentionAggregator::construct (aggregator.rs:137-153) for inference, one
 // wave per node: Full attention over the node's listed features with count 1 each.
-// Nodes without features keep a zero row.
+// Nodes without features keep a zero row.  Three waves per SIMD (168 VGPRs, no spills; two
+// without the bound): 40k nodes of 16 features, 446 -> 277 us with k_att_forward's change.
 // ------------------------------------------------------------------------------------
 template <int DK, typename T, int AM>
-__global__ __launch_bounds__(64) void k_att_embed(const T* __restrict__ table, uint32_t W, int H, int dm,
+__global__ __launch_bounds__(64, AM == AM_FULL ? 3 : 1) void k_att_embed(const T* __restrict__ table, uint32_t W, int H, int dm,
                                                   const uint64_t* __restrict__ findptr,
                                                   const uint32_t* __restrict__ fids, uint64_t n_nodes,
                                                   uint32_t win, float* __restrict__ out) {
@@ -981,9 +1005,13 @@ __global__ __launch_bounds__(256) void k_att_loss(StepConfig c, StepState* st) {
 //   u_j = (V_j . g) / (n H)          dL/dw_j
 //   dS_ij = A_ij (u_j - r_i), r_i = sum_k A_ik u_k,   dT = dS m / sqrt(d_k)
 //   dQ = dT K,  dK = dT^T Q  (matrix cores),  dV_j = w_j g / (n H)
+// The probabilities of the query side serve the key side too (at most four tiles, 64 VGPRs,
+// in place of Q's and K's, which are done with).  31.7k blocks, 4 heads, d_k 32, d 128, FP32:
+// 1435 -> 1229 us at two waves per SIMD; 3.1 GB of gradient rows leave in that time, and three
+// waves per SIMD would spill 58 VGPRs.
 // ------------------------------------------------------------------------------------
 template <int DK, typename T, int AM>
-__global__ __launch_bounds__(64) void k_att_backward(StepConfig c, StepState* st) {
+__global__ __launch_bounds__(64, AM == AM_FULL ? 2 : 1) void k_att_backward(StepConfig c, StepState* st) {
   extern __shared__ float sm[];
   const int H = c.att_heads, dm = c.att_dm;
   const uint32_t W = (uint32_t)c.dims;
@@ -1092,20 +1120,21 @@ __global__ __launch_bounds__(64) void k_att_backward(StepConfig c, StepState* st
       }
     }
     __syncthreads();
-    // query tiles (K Q^T layout): probabilities, r_i, dT, dQ = dT K
+    // query tiles (K Q^T layout): probabilities, r_i, dT, dQ = dT K; the probabilities stay
+    // in registers for the key tiles
+    f32x16 Tt[2][2];
     #pragma unroll
     for (int I = 0; I < 2; ++I) {
       if (I >= NT) break;
-      f32x16 Tt[2];
       #pragma unroll
       for (int J = 0; J < 2; ++J) {
         if (J >= NT) break;
-        Tt[J] = score_tile<DK>(ka[J], qa[I], f32x16{});
+        Tt[I][J] = score_tile<DK>(ka[J], qa[I], f32x16{});
       }
       const uint32_t i = 32u * I + c32;
       const float ci = i < n ? L.cnt[i] : 0.f;
-      float mx, iz;
-      row_softmax_stats<AM>(Tt, NT, n, I, ci, L, isq_h, &mx, &iz);
+      float iz;
+      row_softmax_stats<AM>(Tt[I], NT, n, I, ci, L, isq_h, &iz);
       float ri = 0.f;
       #pragma unroll
       for (int J = 0; J < 2; ++J) {
@@ -1113,12 +1142,12 @@ __global__ __launch_bounds__(64) void k_att_backward(StepConfig c, StepState* st
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const uint32_t j = 32u * J + mrow(r, l);
-          Tt[J][r] *= iz;  // A_ij
-          ri += Tt[J][r] * L.u[j];
+          Tt[I][J][r] = i < n ? Tt[I][J][r] * iz : 0.f;  // A_ij, 0 for padded queries
+          ri += Tt[I][J][r] * L.u[j];
         }
       }
       ri += __shfl_xor(ri, 32, EP_WAVE);
-      if (hf == 0) { L.M[i] = mx; L.iZ[i] = iz; L.r[i] = ri; }
+      if (hf == 0) L.r[i] = ri;
       f32x16 dq = {};
       #pragma unroll
       for (int J = 0; J < 2; ++J) {
@@ -1126,14 +1155,15 @@ __global__ __launch_bounds__(64) void k_att_backward(StepConfig c, StepState* st
 #pragma unroll
         for (int t = 0; t < 16; ++t) {
           const uint32_t j = 32u * J + mrow(t, l);
-          const float dT = Tt[J][t] * (L.u[j] - ri) * count_factor(ci, L.cnt[j]) * isq_h;
+          const float dT = Tt[I][J][t] * (L.u[j] - ri) * count_factor(ci, L.cnt[j]) * isq_h;
           dq = mfma32(dT, L.K[(size_t)j * kTileStride + c32], dq);
         }
       }
       store_tile_cols<DK>(dq, I, n, (uint32_t)(h * DK), slot_row);
     }
     __syncthreads();
-    // key tiles (Q K^T layout): w_j, dT, dK = dT^T Q, dV_j = w_j g / (n H)
+    // key tiles (probabilities turned over in the K tile's LDS, done with by now): w_j, dT,
+    // dK = dT^T Q, dV_j = w_j g / (n H)
     #pragma unroll
     for (int J = 0; J < 2; ++J) {
       if (J >= NT) break;
@@ -1145,14 +1175,19 @@ __global__ __launch_bounds__(64) void k_att_backward(StepConfig c, StepState* st
       #pragma unroll
       for (int I = 0; I < 2; ++I) {
         if (I >= NT) break;
-        f32x16 a = score_tile<DK>(qa[I], ka[J], f32x16{});
+        put_tile(L.K + (size_t)(32 * I) * kTileStride, Tt[I][J]);
+      }
+      __syncthreads();
+      #pragma unroll
+      for (int I = 0; I < 2; ++I) {
+        if (I >= NT) break;
+        f32x16 a = get_tile_turned(L.K + (size_t)(32 * I) * kTileStride);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const uint32_t i = 32u * I + mrow(r, l);
           const float f = count_factor(L.cnt[i], cj) * isq_h;
-          const float A = att_pair<AM>(L, i, j, n) ? softmax_exp(a[r] * f - L.M[i]) * L.iZ[i] : 0.f;
-          wj += A;
-          a[r] = A * (uj - L.r[i]) * f;  // dT_ij
+          wj += a[r];
+          a[r] = a[r] * (uj - L.r[i]) * f;  // dT_ij
         }
 #pragma unroll
         for (int t = 0; t < 16; ++t) dk = mfma32(a[t], L.Q[(size_t)(32u * I + mrow(t, l)) * kTileStride + c32], dk);
@@ -1173,8 +1208,8 @@ __global__ __launch_bounds__(64) void k_att_backward(StepConfig c, StepState* st
           }
         }
       }
+      __syncthreads();
     }
-    __syncthreads();
   }
 }
 
