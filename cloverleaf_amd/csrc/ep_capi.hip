@@ -64,7 +64,8 @@ void shuffle(std::vector<T>& v, HostRng& r) {
 // threads move filled ones out, taking the page faults of a fresh array side by side.  The
 // runtime's own pageable copy waits for the faults and the transfer in turn: 51 MB into a fresh
 // array take it 5.2 ms on a MI355X host and 3.0 into a touched one, the transfer alone 1.0;
-// this takes 1.6.  The ring (8 MB) belongs to one context or aligner, from its first large
+// this takes 1.6.  Starting the threads costs about what 10 MB gain: a call with 8.4 MB of
+// results took 0.2 ms longer this way, with 10 MB 0.1, with 15 MB 0.4 less.  The ring (8 MB) belongs to one context or aligner, from its first large
 // copy to its end; the threads end with the copy.
 class HostCopy {
  public:
@@ -78,13 +79,16 @@ class HostCopy {
   }
 
   hipError_t run(void* dst, const void* src, size_t bytes, hipStream_t s) {
-    if (bytes >= kMinBytes && prepare() && start()) return copy((unsigned char*)dst, (const unsigned char*)src, bytes, s);
+    // a second thread reading from the same context meanwhile takes the runtime's copy
+    std::unique_lock<std::mutex> own(use_, std::try_to_lock);
+    if (bytes >= kMinBytes && own && prepare() && start()) return copy((unsigned char*)dst, (const unsigned char*)src, bytes, s);
+    if (own) own.unlock();
     hipError_t e = bytes ? hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s) : hipSuccess;
     return e == hipSuccess ? hipStreamSynchronize(s) : e;
   }
 
  private:
-  static constexpr size_t kMinBytes = (size_t)8 << 20, kChunk = (size_t)1 << 20;
+  static constexpr size_t kMinBytes = (size_t)12 << 20, kChunk = (size_t)1 << 20;
   static constexpr int kRing = 8, kFlight = 3, kThreads = 6;  // chunks, copies in flight, threads
 
   // The ring and its events; false when they are not to be had.
@@ -173,6 +177,7 @@ class HostCopy {
   unsigned char* ring_ = nullptr;
   hipEvent_t ev_[kRing] = {};
   std::thread threads_[kThreads];
+  std::mutex use_;  // the ring and the threads, for one copy
   std::mutex mu_;
   std::condition_variable cv_;
   unsigned char* dst_ = nullptr;
