@@ -2751,8 +2751,13 @@ __device__ inline void add_named_rows(const StepConfig& c, const RowNames<H>& na
     for (int u = 0; u < U; ++u) {
       const uint32_t t = min(t0 + (uint32_t)u, last);
       load_packed_f16<D>(c.adjh + (size_t)lane_value(names.slot, t) * D, lane, w[u]);
-      const float s = __uint_as_float(lane_value(__float_as_uint(names.scale), t));
-      sc[u] = (uint32_t)u < n ? s : 0.f;  // rows past n count as zero (FP16 rows are finite)
+      sc[u] = __uint_as_float(lane_value(__float_as_uint(names.scale), t));
+    }
+    if (n < (uint32_t)U) {  // rows past n count as zero, also where the last row is infinite
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int p = 0; p < PW; ++p) w[u][p] = (uint32_t)u < n ? w[u][p] : 0u;
     }
     float r[U / 2][PL];
 #pragma unroll
