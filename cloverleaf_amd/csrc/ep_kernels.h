@@ -47,16 +47,16 @@ struct StepHead {
   uint32_t reg_next;       // next plan region for k_seg_update (cleared by k_seg_plan)
 };
 
-// Sort grids of up to kSortGroups x kSortGroupBlocks blocks keep digit totals per group of
-// blocks (see k_rs_scatter).
-constexpr uint32_t kSortGroups = 16u, kSortGroupBlocks = 16u;
+// The radix sort keeps digit totals per group of consecutive blocks (see k_rs_scatter): 16
+// groups for grids of up to 256 blocks, 32 for larger ones.
+constexpr uint32_t kSortGroupsMax = 32u;
+__host__ __device__ inline uint32_t sort_groups(int grid) { return grid <= 256 ? 16u : kSortGroupsMax; }
 
 // The device's state: the values above (what the host reads back) and the tables.
 struct StepState : StepHead {
-  uint32_t dtot[4][2048];  // radix-sort digit totals, one row per sort pass (<= 11-bit digits)
-  // digit totals of groups of sort blocks, kSortGroups tables per pass (at most 2 passes of
+  // digit totals of groups of sort blocks, a table per group and pass (at most 2 passes of
   // 11-bit or 3 of 9-bit digits)
-  uint32_t dgrp[2 * kSortGroups * 2048];
+  uint32_t dgrp[2 * kSortGroupsMax * 2048];
   // cumulative rows updated, one slot per block of the row kernels: by the short-row kernel,
   // and by the medium- and long-row kernels (stat_unique: by the atomic path)
   unsigned long long upd_short[2048], upd_long[2048];
@@ -180,8 +180,7 @@ struct StepConfig {
   uint32_t key_cap;
   uint32_t* ghist;         // [2048 * sort_grid]
   int sort_grid;
-  int sort_groups;         // k_sample clears dgrp (1) or dtot (0), sort_totals words of it (set by
-  uint32_t sort_totals;    // launch_sample)
+  uint32_t sort_totals;    // words of dgrp that k_sample clears (set by launch_sample)
   // scatter (sort path)
   float* G;                // [key_cap*D] compact gradient rows (bounded by unique count)
   uint32_t* ufeat;         // [key_cap]

@@ -489,9 +489,7 @@ __device__ inline uint32_t nth_set_bit(uint64_t m, uint32_t q) {
 // anchors from the cursor themselves, so the step needs no launch of its own for it.
 __global__ __launch_bounds__(256) void k_sample(StepConfig c, StepState* st, float lr_override) {
   const int lane = threadIdx.x & 63;
-  // the sort's totals: of the whole grid (k_rs_scan's) or of its groups, whichever it uses
-  uint32_t* totals = c.sort_groups ? st->dgrp : &st->dtot[0][0];
-  for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < c.sort_totals; i += gridDim.x * 256u) totals[i] = 0u;
+  for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < c.sort_totals; i += gridDim.x * 256u) st->dgrp[i] = 0u;
   if (blockIdx.x == gridDim.x - 1u) {
     begin_step(c, st, lr_override);
     return;
@@ -1690,9 +1688,10 @@ __device__ inline uint64_t digit_peers(bool act, uint32_t d) {
 
 // Pass 0 reads the emitted keys (st->n_keys, sentinels included) and drops the sentinels;
 // later passes read the st->n_real compacted keys.
-// GROUPS: also the totals of groups of kSortGroupBlocks blocks, for a k_rs_scatter that works
-// out its digit bases itself.
-template <int RB, bool GROUPS>
+// Besides its own counts a block adds them to its group's totals.  Totals of the whole grid
+// took one table: at 20 ns per block and line of it (blocks of all XCDs), 31 us of a pass at
+// 1536 blocks.
+template <int RB>
 __global__ __launch_bounds__(256) void k_rs_hist(const uint32_t* __restrict__ kin, StepState* st, uint32_t* ghist,
                                                  int pass, int shift, int G, uint32_t sent) {
   constexpr uint32_t BINS = 1u << RB, MASK = BINS - 1u;
@@ -1700,7 +1699,7 @@ __global__ __launch_bounds__(256) void k_rs_hist(const uint32_t* __restrict__ ki
   const int tid = threadIdx.x, lane = tid & 63;
   uint32_t lo, hi;
   block_range(pass == 0 ? st->n_keys : st->n_real, G, blockIdx.x, &lo, &hi);
-  if (GROUPS && lo >= hi) return;  // k_rs_scatter reads the counts of blocks with elements only
+  if (lo >= hi) return;  // k_rs_scatter reads the counts of blocks with elements only
   for (uint32_t d = tid; d < BINS; d += 256u) h[d] = 0u;
   __syncthreads();
   for (uint32_t t0 = lo; t0 < hi; t0 += 256u * RS_ITEMS) {
@@ -1727,49 +1726,11 @@ __global__ __launch_bounds__(256) void k_rs_hist(const uint32_t* __restrict__ ki
     }
   }
   __syncthreads();
+  const uint32_t ng = sort_groups(G), gsize = ((uint32_t)G + ng - 1u) / ng;
+  uint32_t* tot = st->dgrp + ((uint32_t)pass * ng + blockIdx.x / gsize) * BINS;
   for (uint32_t d = tid; d < BINS; d += 256u) {
     ghist[(size_t)blockIdx.x * BINS + d] = h[d];  // block-major: coalesced
-    uint32_t* tot = GROUPS ? &st->dgrp[((uint32_t)pass * kSortGroups + blockIdx.x / kSortGroupBlocks) * BINS + d]
-                           : &st->dtot[pass][d];
-    if (h[d]) atomicAdd(tot, h[d]);
-  }
-}
-
-// Grids of up to kSortGroups x kSortGroupBlocks blocks (steps of up to 2M keys at capacity):
-// every scatter block adds up its bases from the group totals and its group's counts, at most
-// 32 coalesced reads per digit, instead of a k_rs_scan launch between the two kernels (6.6 of
-// 17 us of a pass at 16k keys on MI355X; at 2048 blocks the reads would cost what the scan
-// does).
-//
-// Turns the block-major counts into scatter bases: base(blk, d) = sum_{d' < d} total(d')
-// + sum_{b < blk} count(b, d).  One wave per digit; lane l owns G/64 consecutive source
-// blocks (their loads are independent), then a wave scan.
-template <int RB>
-__global__ __launch_bounds__(256) void k_rs_scan(uint32_t* ghist, StepState* st, int pass, int G) {
-  constexpr uint32_t BINS = 1u << RB;
-  const int lane = threadIdx.x & 63;
-  const uint32_t d = blockIdx.x * NW + (threadIdx.x >> 6);
-  if (d >= BINS) return;
-  uint32_t pre = 0;
-  for (uint32_t q = lane; q < d; q += 64u) pre += st->dtot[pass][q];
-  pre = wave_sum_u32(pre);
-  if (d == BINS - 1u && lane == 0) st->n_real = pre + st->dtot[pass][d];
-  const uint32_t per = (uint32_t)G / 64u;  // G is a multiple of 256
-  const uint32_t b0 = (uint32_t)lane * per;
-  uint32_t loc = 0;
-  for (uint32_t i = 0; i < per; ++i) loc += ghist[(size_t)(b0 + i) * BINS + d];
-  uint32_t inc = loc;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t y = __shfl_up(inc, off, EP_WAVE);
-    if (lane >= off) inc += y;
-  }
-  uint32_t run = pre + inc - loc;
-  for (uint32_t i = 0; i < per; ++i) {
-    const size_t idx = (size_t)(b0 + i) * BINS + d;
-    const uint32_t x = ghist[idx];
-    ghist[idx] = run;
-    run += x;
+    if (h[d]) atomicAdd(&tot[d], h[d]);
   }
 }
 
@@ -1780,9 +1741,16 @@ __global__ __launch_bounds__(256) void k_rs_scan(uint32_t* ghist, StepState* st,
 // order, so each digit's elements leave as one contiguous run instead of one scattered
 // store each.  Stable: the tile order is (wave, item, lane) = element order, and tiles
 // and blocks follow each other through the per-block digit bases.
+//
+// A block adds its bases up itself, base(d) = sum_{d' < d} total(d') + sum_{b < blk} count(b, d),
+// from the totals of the groups and the counts of its own group's blocks before it: 16 tables
+// and up to 15 counts per digit at 256 blocks, 32 and up to 47 at 1536, coalesced, on a
+// device that a scan kernel between the two would leave nearly idle.  A pass with it, totals in
+// one table, against one without on MI355X: 8.8M keys (1536 blocks) 105 against 63 us, 4.1M
+// (768) 62 against 39; at 16k keys 17 against 10.
 static constexpr int RS_SCATTER_ITEMS = 16;
 
-template <int RB, bool GROUPS>
+template <int RB>
 __global__ __launch_bounds__(256) void k_rs_scatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
                                                     uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
                                                     StepState* st, const uint32_t* __restrict__ ghist, int pass,
@@ -1790,7 +1758,6 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const uint32_t* __restrict__
   constexpr uint32_t BINS = 1u << RB, MASK = BINS - 1u;
   constexpr int IT = RS_SCATTER_ITEMS;
   constexpr uint32_t TILE = 256u * IT;
-  constexpr uint32_t WSPAN = 64u * IT;                          // elements of one wave in a tile
   constexpr uint32_t DPT = BINS >= 256u ? BINS / 256u : 1u;     // digits per thread in the scans
   __shared__ uint32_t run[BINS];       // output position of the block's next element of each digit
   __shared__ uint32_t wcnt[NW][BINS];  // per-wave digit counts, then their prefix over the waves
@@ -1800,60 +1767,61 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const uint32_t* __restrict__
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   uint32_t lo, hi;
   block_range(pass == 0 ? st->n_keys : st->n_real, G, blockIdx.x, &lo, &hi);
-  if (GROUPS && lo >= hi) return;
-  if constexpr (GROUPS) {
-    // base(d) = totals of the smaller digits + counts of d in the blocks before this one:
-    // thread tid owns digits [tid*DPT, tid*DPT + DPT)
-    const uint32_t grp = blockIdx.x / kSortGroupBlocks;
-    const uint32_t* gs = st->dgrp + (uint32_t)pass * kSortGroups * BINS;
+  if (lo >= hi) return;
+  {
+    // thread tid owns digits [tid * DPT, tid * DPT + DPT)
+    const uint32_t ng = sort_groups(G), gsize = ((uint32_t)G + ng - 1u) / ng, grp = blockIdx.x / gsize;
+    const uint32_t d0 = (uint32_t)tid * DPT;
+    const uint32_t* gs = st->dgrp + (uint32_t)pass * ng * BINS + d0;
     uint32_t bef[DPT], tot[DPT], tsum = 0u;
 #pragma unroll
-    for (uint32_t j = 0; j < DPT; ++j) {
-      const uint32_t d = (uint32_t)tid * DPT + j;
-      bef[j] = tot[j] = 0u;
-      if (d < BINS) {
+    for (uint32_t j = 0; j < DPT; ++j) bef[j] = tot[j] = 0u;
+    if (d0 < BINS) {
+#pragma unroll 16
+      for (uint32_t q = 0; q < ng; ++q)
 #pragma unroll
-        for (uint32_t q = 0; q < kSortGroups; ++q) {
-          const uint32_t x = gs[q * BINS + d];
+        for (uint32_t j = 0; j < DPT; ++j) {
+          const uint32_t x = gs[q * BINS + j];
           tot[j] += x;
           bef[j] += q < grp ? x : 0u;
         }
-        for (uint32_t b = grp * kSortGroupBlocks; b < blockIdx.x; ++b) bef[j] += ghist[(size_t)b * BINS + d];
-      }
-      tsum += tot[j];
+#pragma unroll 8
+      for (uint32_t b = grp * gsize; b < blockIdx.x; ++b)
+#pragma unroll
+        for (uint32_t j = 0; j < DPT; ++j) bef[j] += ghist[(size_t)b * BINS + d0 + j];
     }
+#pragma unroll
+    for (uint32_t j = 0; j < DPT; ++j) tsum += tot[j];
     uint32_t all = 0u;
     uint32_t start = block_exclusive_scan(tsum, s_wave, &all);
     if (blockIdx.x == 0u && tid == 0 && pass == 0) st->n_real = all;
 #pragma unroll
     for (uint32_t j = 0; j < DPT; ++j) {
-      const uint32_t d = (uint32_t)tid * DPT + j;
-      if (d < BINS) run[d] = start + bef[j];
+      if (d0 < BINS) run[d0 + j] = start + bef[j];
       start += tot[j];
     }
   }
   for (uint32_t d = tid; d < BINS; d += 256u) {
-    if constexpr (!GROUPS) run[d] = ghist[(size_t)blockIdx.x * BINS + d];
 #pragma unroll
     for (int q = 0; q < NW; ++q) wcnt[q][d] = 0u;
   }
   __syncthreads();
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   // a block of a small step holds less than a tile: its waves share what there is
-  const uint32_t span = GROUPS ? (min(hi - lo, TILE) + 255u) / 256u * 64u : WSPAN;
+  const uint32_t span = (min(hi - lo, TILE) + 255u) / 256u * 64u;
   for (uint32_t t0 = lo; t0 < hi; t0 += TILE) {
     uint32_t k[IT], val[IT], rk[IT];
 #pragma unroll
     for (int q = 0; q < IT; ++q) {
       const uint32_t i = t0 + (uint32_t)w * span + (uint32_t)q * 64u + (uint32_t)lane;
-      const bool in = (!GROUPS || (uint32_t)q * 64u < span) && i < hi;
+      const bool in = (uint32_t)q * 64u < span && i < hi;
       k[q] = in ? kin[i] : sent;  // sent: inactive (pass 0 drops the sentinels)
       val[q] = in ? vin[i] : 0u;
     }
     // ranks within the wave's quarter: count of earlier elements with the same digit
 #pragma unroll
     for (int q = 0; q < IT; ++q) {
-      if (GROUPS && (uint32_t)q * 64u >= span) break;
+      if ((uint32_t)q * 64u >= span) break;
       const bool act = k[q] != sent;
       const uint32_t d = (k[q] >> shift) & MASK;
       // the lanes sharing this lane's digit: all active lanes when the wave holds one digit
@@ -3318,8 +3286,7 @@ hipError_t launch_sample(const StepConfig& c0, StepState* st, float lr, hipStrea
   StepConfig c = c0;
   int passes, rb;
   radix_plan(c.sort_bits, &passes, &rb);
-  c.sort_groups = c.sort_grid <= (int)(kSortGroups * kSortGroupBlocks);
-  c.sort_totals = !c.train ? 0u : c.sort_groups ? ((uint32_t)passes * kSortGroups) << rb : 4u * 2048u;
+  c.sort_totals = c.train ? ((uint32_t)passes * sort_groups(c.sort_grid)) << rb : 0u;
   hipLaunchKernelGGL(k_sample, dim3((c.batch + NW - 1) / NW + 1), dim3(256), (size_t)NW * c.S * sizeof(uint32_t), s, c, st,
                      lr);
   return hipGetLastError();
@@ -3385,30 +3352,21 @@ static int resident_blocks(int cap) {
   return n < cap ? n : cap;
 }
 
-template <int RB, bool GROUPS>
-static void launch_sort_passes(const StepConfig& c, StepState* st, hipStream_t s, int passes, int* cur) {
+template <int RB>
+static void launch_sort_rb(const StepConfig& c, StepState* st, hipStream_t s, int passes, int* cur) {
+  static_assert(kSortGroupsMax << RB <= sizeof(StepState::dgrp) / sizeof(uint32_t) / (RB <= 9 ? 3 : 2), "a table per pass");
   // whole rounds of resident scatter blocks (at 9-bit digits its tile and counters take
   // 44 KB of LDS, three blocks per CU): a last, partial round would leave part of the
-  // device idle; the three kernels of a pass share the block partition
-  const int res = resident_blocks<k_rs_scatter<RB, GROUPS>>(c.sort_grid);
+  // device idle; the two kernels of a pass share the block partition
+  const int res = resident_blocks<k_rs_scatter<RB>>(c.sort_grid);
   const int G = res < c.sort_grid ? (c.sort_grid / res) * res : c.sort_grid;
   for (int p = 0; p < passes; ++p) {
     const int shift = p * RB;
-    hipLaunchKernelGGL((k_rs_hist<RB, GROUPS>), dim3(G), dim3(256), 0, s, c.keys[*cur], st, c.ghist, p, shift, G,
-                       c.sentinel);
-    if constexpr (!GROUPS)
-      hipLaunchKernelGGL((k_rs_scan<RB>), dim3(((1u << RB) + NW - 1u) / NW), dim3(256), 0, s, c.ghist, st, p, G);
-    hipLaunchKernelGGL((k_rs_scatter<RB, GROUPS>), dim3(G), dim3(256), 0, s, c.keys[*cur], c.slots[*cur],
-                       c.keys[1 - *cur], c.slots[1 - *cur], st, c.ghist, p, shift, G, c.sentinel);
+    hipLaunchKernelGGL((k_rs_hist<RB>), dim3(G), dim3(256), 0, s, c.keys[*cur], st, c.ghist, p, shift, G, c.sentinel);
+    hipLaunchKernelGGL((k_rs_scatter<RB>), dim3(G), dim3(256), 0, s, c.keys[*cur], c.slots[*cur], c.keys[1 - *cur],
+                       c.slots[1 - *cur], st, c.ghist, p, shift, G, c.sentinel);
     *cur = 1 - *cur;
   }
-}
-
-template <int RB>
-static void launch_sort_rb(const StepConfig& c, StepState* st, hipStream_t s, int passes, int* cur) {
-  static_assert(kSortGroups << RB <= sizeof(StepState::dgrp) / sizeof(uint32_t) / (RB <= 9 ? 3 : 2), "a table per pass");
-  if (c.sort_grid <= (int)(kSortGroups * kSortGroupBlocks)) launch_sort_passes<RB, true>(c, st, s, passes, cur);
-  else launch_sort_passes<RB, false>(c, st, s, passes, cur);
 }
 
 hipError_t launch_sort(const StepConfig& c, StepState* st, hipStream_t s, int* out_buf) {

@@ -1,8 +1,8 @@
-"""The radix sort's two base computations: scatter blocks that add up their digit bases from
-group totals (steps of up to 2M keys at capacity) and the scan kernel of larger grids, at
-every digit width class: one pass (up to 11 bits), two passes of 8 to 11 bits, three passes.
-The same batch on contexts of either capacity updates the table, moments and loss alike, bit
-for bit, and the merged gradient matches the FP64 oracle's feature set."""
+"""The radix sort's scatter blocks add up their digit bases from the totals of groups of
+blocks: 16 groups of up to 16 blocks (steps of up to 2M keys at capacity) and 32 larger
+groups, at every digit width class: one pass (up to 11 bits), two passes of 8 to 11 bits,
+three passes.  The same batch on contexts of either capacity updates the table, moments and
+loss alike, bit for bit, and the merged gradient matches the FP64 oracle's feature set."""
 import numpy as np
 import pytest
 
