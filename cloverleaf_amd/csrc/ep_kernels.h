@@ -2,6 +2,7 @@
 // (ep_kernels.hip).  Not part of the public C ABI.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 namespace ep {
@@ -46,6 +47,9 @@ struct StepHead {
   uint32_t n_real;         // non-sentinel keys (the sorted key count)
   uint32_t reg_next;       // next plan region for k_seg_update (cleared by k_seg_plan)
 };
+
+static_assert(offsetof(StepHead, n_long) % 8 == 0 && offsetof(StepHead, n_pieces) == offsetof(StepHead, n_long) + 4,
+              "k_seg_plan adds to both in one 64-bit atomic");
 
 // The radix sort keeps digit totals per group of consecutive blocks (see k_rs_scatter): 16
 // groups for grids of up to 256 blocks, 32 for larger ones.

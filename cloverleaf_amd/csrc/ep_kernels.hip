@@ -97,6 +97,22 @@ __device__ inline uint32_t wave_lower_bound(const uint32_t* __restrict__ K, uint
   return lo;
 }
 
+// The same for an end that is near more often than not: samples 64 entries apart first, then
+// 4096, then over the whole rest, so that a row of up to 4096 entries takes two dependent
+// loads instead of the four of a search over millions of keys.
+__device__ inline uint32_t wave_row_end(const uint32_t* __restrict__ K, uint32_t lo, uint32_t hi, uint32_t x) {
+  const uint32_t lane = lane_id();
+  for (uint32_t step = 64u; step <= 4096u && hi > lo && hi - lo > 64u * step; step *= 64u) {
+    const uint64_t m = __ballot(K[lo + lane * step] >= x);
+    if (m) {
+      const uint32_t f = (uint32_t)(__ffsll((unsigned long long)m) - 1);
+      return f == 0u ? lo : wave_lower_bound(K, lo + (f - 1u) * step + 1u, lo + f * step, x);
+    }
+    lo += 63u * step + 1u;
+  }
+  return wave_lower_bound(K, lo, hi, x);
+}
+
 // Accumulate rows table[fids[fs..fe)] into acc (lane slice), U row loads in flight.
 template <int D, int U, typename T>
 __device__ inline void gather_rows(const T* __restrict__ table, const uint32_t* __restrict__ fids,
@@ -2266,7 +2282,7 @@ __global__ __launch_bounds__(256) void k_seg_plan(StepConfig c, StepState* st, c
     if (find) {
       // the end of the row that fills the rest of the window (both search paths share this
       // one call); the chunks before the one holding it start no row
-      const uint32_t hi = wave_lower_bound(Ks, i0 + 128u, n, find);
+      const uint32_t hi = wave_row_end(Ks, i0 + 128u, n, find);
       if (hi / 64u > chunk + 1u) jump = min(hi / 64u, cend);
       if (deferred) {
         // the chunk's last row runs past the window: register it as long, its runs found by
@@ -2281,13 +2297,12 @@ __global__ __launch_bounds__(256) void k_seg_plan(StepConfig c, StepState* st, c
           if (bnd(b + 1) > bnd(b)) ++nr;
           pcs += long_run_pieces(bnd(b + 1) - bnd(b));
         }
-        uint32_t idx = 0, pb = 0;
-        if (lane == 0) {
-          idx = atomicAdd(&st->n_long, 1u);
-          pb = atomicAdd(&st->n_pieces, pcs);
-        }
-        idx = (uint32_t)__builtin_amdgcn_readfirstlane((int)idx);
-        pb = (uint32_t)__builtin_amdgcn_readfirstlane((int)pb);
+        // n_long and n_pieces in one returning atomic: every hot row waits for its turn there
+        unsigned long long at = 0ull;
+        if (lane == 0)
+          at = atomicAdd(reinterpret_cast<unsigned long long*>(&st->n_long), (unsigned long long)pcs << 32 | 1ull);
+        const uint32_t idx = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at);
+        const uint32_t pb = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32));
         if (idx < c.long_cap) {
           auto run_at = [&](uint32_t j, uint32_t* a, uint32_t* z, uint32_t* bq) {
             uint32_t k = 0, seen = 0;  // j-th nonempty batch run
