@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <cstring>
 #include <iterator>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <thread>
@@ -458,6 +459,7 @@ int place_step_buffers(ep_ctx* c, uint32_t batch, ep::StepConfig& b, Place&& pla
     EP_TRY(place(&b.slots[i], keycap));
   }
   EP_TRY(place(&b.ghist, (size_t)2048 * sort_grid));
+  EP_TRY(place(&b.dgrp, ep::kSortTotals));
   EP_TRY(place(&b.long_st, long_cap));
   EP_TRY(place(&b.long_len, long_cap));
   EP_TRY(place(&b.long_pbase, long_cap));
@@ -1035,12 +1037,10 @@ int ep_create(const ep_config* cfg, ep_ctx** out) {
   int r = c->alloc(&c->d_state, 1);
   if (r == EP_OK) r = c->alloc(&c->d_vstate, 1);
   if (r != EP_OK) { delete c; return r; }
-  ep::StepHead head{};
-  head.next_step = 1;
-  for (ep::StepState* st : {c->d_state, c->d_vstate}) {
-    if (e == hipSuccess) e = hipMemset(st, 0, sizeof(*st));
-    if (e == hipSuccess) e = hipMemcpy(st, &head, sizeof(head), hipMemcpyHostToDevice);
-  }
+  const std::unique_ptr<ep::StepState> zero(new ep::StepState());
+  zero->next_step = 1;
+  e = hipMemcpy(c->d_state, zero.get(), sizeof(*zero), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(c->d_vstate, zero.get(), sizeof(*zero), hipMemcpyHostToDevice);
   if (e != hipSuccess) { delete c; return fail(EP_EHIP, std::string("hipMemcpy: ") + hipGetErrorString(e)); }
   *out = c;
   return EP_OK;

@@ -54,13 +54,13 @@ static_assert(offsetof(StepHead, n_long) % 8 == 0 && offsetof(StepHead, n_pieces
 // The radix sort keeps digit totals per group of consecutive blocks (see k_rs_scatter): 16
 // groups for grids of up to 256 blocks, 32 for larger ones.
 constexpr uint32_t kSortGroupsMax = 32u;
+// Words of the totals: a table per group and pass (at most 2 passes of 11-bit or 3 of 9-bit
+// digits).
+constexpr uint32_t kSortTotals = 2u * kSortGroupsMax * 2048u;
 __host__ __device__ inline uint32_t sort_groups(int grid) { return grid <= 256 ? 16u : kSortGroupsMax; }
 
 // The device's state: the values above (what the host reads back) and the tables.
 struct StepState : StepHead {
-  // digit totals of groups of sort blocks, a table per group and pass (at most 2 passes of
-  // 11-bit or 3 of 9-bit digits)
-  uint32_t dgrp[2 * kSortGroupsMax * 2048];
   // cumulative rows updated, one slot per block of the row kernels: by the short-row kernel,
   // and by the medium- and long-row kernels (stat_unique: by the atomic path)
   unsigned long long upd_short[2048], upd_long[2048];
@@ -183,6 +183,7 @@ struct StepConfig {
   uint32_t* slots[2];
   uint32_t key_cap;
   uint32_t* ghist;         // [2048 * sort_grid]
+  uint32_t* dgrp;          // [kSortTotals] digit totals of groups of sort blocks
   int sort_grid;
   uint32_t sort_totals;    // words of dgrp that k_sample clears (set by launch_sample)
   // scatter (sort path)

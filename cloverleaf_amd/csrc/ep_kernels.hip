@@ -226,7 +226,7 @@ __device__ inline uint32_t hash_lookup(const uint32_t* h, uint32_t mask, uint32_
 }
 
 // ------------------------------------------------------------------------------------
-// k_step_begin: advance the batch cursor, LR schedule and Adam bias corrections.
+// begin_step: batch cursor, LR schedule and Adam bias corrections (k_sample, last block).
 // LRScheduler::cos_decay (scheduler.rs:39-47) as built at mod.rs:132-137, in f32.
 // ------------------------------------------------------------------------------------
 __device__ inline float scheduled_lr(const StepConfig& c, uint64_t cur) {
@@ -505,7 +505,7 @@ __device__ inline uint32_t nth_set_bit(uint64_t m, uint32_t q) {
 // anchors from the cursor themselves, so the step needs no launch of its own for it.
 __global__ __launch_bounds__(256) void k_sample(StepConfig c, StepState* st, float lr_override) {
   const int lane = threadIdx.x & 63;
-  for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < c.sort_totals; i += gridDim.x * 256u) st->dgrp[i] = 0u;
+  for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < c.sort_totals; i += gridDim.x * 256u) c.dgrp[i] = 0u;
   if (blockIdx.x == gridDim.x - 1u) {
     begin_step(c, st, lr_override);
     return;
@@ -1708,7 +1708,7 @@ __device__ inline uint64_t digit_peers(bool act, uint32_t d) {
 // took one table: at 20 ns per block and line of it (blocks of all XCDs), 31 us of a pass at
 // 1536 blocks.
 template <int RB>
-__global__ __launch_bounds__(256) void k_rs_hist(const uint32_t* __restrict__ kin, StepState* st, uint32_t* ghist,
+__global__ __launch_bounds__(256) void k_rs_hist(const uint32_t* __restrict__ kin, StepState* st, uint32_t* ghist, uint32_t* dgrp,
                                                  int pass, int shift, int G, uint32_t sent) {
   constexpr uint32_t BINS = 1u << RB, MASK = BINS - 1u;
   __shared__ uint32_t h[BINS];
@@ -1743,7 +1743,7 @@ __global__ __launch_bounds__(256) void k_rs_hist(const uint32_t* __restrict__ ki
   }
   __syncthreads();
   const uint32_t ng = sort_groups(G), gsize = ((uint32_t)G + ng - 1u) / ng;
-  uint32_t* tot = st->dgrp + ((uint32_t)pass * ng + blockIdx.x / gsize) * BINS;
+  uint32_t* tot = dgrp + ((uint32_t)pass * ng + blockIdx.x / gsize) * BINS;
   for (uint32_t d = tid; d < BINS; d += 256u) {
     ghist[(size_t)blockIdx.x * BINS + d] = h[d];  // block-major: coalesced
     if (h[d]) atomicAdd(&tot[d], h[d]);
@@ -1769,7 +1769,8 @@ static constexpr int RS_SCATTER_ITEMS = 16;
 template <int RB>
 __global__ __launch_bounds__(256) void k_rs_scatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
                                                     uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
-                                                    StepState* st, const uint32_t* __restrict__ ghist, int pass,
+                                                    StepState* st, const uint32_t* __restrict__ ghist,
+                                                    const uint32_t* __restrict__ dgrp, int pass,
                                                     int shift, int G, uint32_t sent) {
   constexpr uint32_t BINS = 1u << RB, MASK = BINS - 1u;
   constexpr int IT = RS_SCATTER_ITEMS;
@@ -1788,7 +1789,7 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const uint32_t* __restrict__
     // thread tid owns digits [tid * DPT, tid * DPT + DPT)
     const uint32_t ng = sort_groups(G), gsize = ((uint32_t)G + ng - 1u) / ng, grp = blockIdx.x / gsize;
     const uint32_t d0 = (uint32_t)tid * DPT;
-    const uint32_t* gs = st->dgrp + (uint32_t)pass * ng * BINS + d0;
+    const uint32_t* gs = dgrp + (uint32_t)pass * ng * BINS + d0;
     uint32_t bef[DPT], tot[DPT], tsum = 0u;
 #pragma unroll
     for (uint32_t j = 0; j < DPT; ++j) bef[j] = tot[j] = 0u;
@@ -3369,7 +3370,7 @@ static int resident_blocks(int cap) {
 
 template <int RB>
 static void launch_sort_rb(const StepConfig& c, StepState* st, hipStream_t s, int passes, int* cur) {
-  static_assert(kSortGroupsMax << RB <= sizeof(StepState::dgrp) / sizeof(uint32_t) / (RB <= 9 ? 3 : 2), "a table per pass");
+  static_assert(kSortGroupsMax << RB <= kSortTotals / (RB <= 9 ? 3 : 2), "a table per pass");
   // whole rounds of resident scatter blocks (at 9-bit digits its tile and counters take
   // 44 KB of LDS, three blocks per CU): a last, partial round would leave part of the
   // device idle; the two kernels of a pass share the block partition
@@ -3377,9 +3378,10 @@ static void launch_sort_rb(const StepConfig& c, StepState* st, hipStream_t s, in
   const int G = res < c.sort_grid ? (c.sort_grid / res) * res : c.sort_grid;
   for (int p = 0; p < passes; ++p) {
     const int shift = p * RB;
-    hipLaunchKernelGGL((k_rs_hist<RB>), dim3(G), dim3(256), 0, s, c.keys[*cur], st, c.ghist, p, shift, G, c.sentinel);
+    hipLaunchKernelGGL((k_rs_hist<RB>), dim3(G), dim3(256), 0, s, c.keys[*cur], st, c.ghist, c.dgrp, p, shift, G,
+                       c.sentinel);
     hipLaunchKernelGGL((k_rs_scatter<RB>), dim3(G), dim3(256), 0, s, c.keys[*cur], c.slots[*cur], c.keys[1 - *cur],
-                       c.slots[1 - *cur], st, c.ghist, p, shift, G, c.sentinel);
+                       c.slots[1 - *cur], st, c.ghist, c.dgrp, p, shift, G, c.sentinel);
     *cur = 1 - *cur;
   }
 }
