@@ -534,7 +534,7 @@ void clear_step_buffers(ep::StepConfig& b) {
   b.nbr_w = nullptr; b.nbroff = nullptr; b.nbr_sel = nullptr; b.nbr_selw = nullptr;
   b.adj = nullptr; b.adjh = nullptr; b.ascale = nullptr; b.coef = nullptr; b.elig = nullptr; b.loss = nullptr;
   b.pass_loss = nullptr; b.xout = nullptr;
-  b.keys[0] = b.keys[1] = nullptr; b.slots[0] = b.slots[1] = nullptr; b.ghist = nullptr;
+  b.keys[0] = b.keys[1] = nullptr; b.slots[0] = b.slots[1] = nullptr; b.ghist = nullptr; b.dgrp = nullptr;
   b.G = nullptr; b.ufeat = nullptr;
   b.srec = nullptr; b.mrec = nullptr; b.scount = nullptr; b.mcount = nullptr;
   b.long_st = nullptr; b.long_len = nullptr; b.long_pbase = nullptr; b.long_runs = nullptr; b.long_rlen = nullptr;
@@ -562,7 +562,7 @@ int ensure_step_buffers(ep_ctx* c, uint32_t batch) {
   c->release(b.adj); c->release(b.adjh); c->release(b.ascale); c->release(b.coef); c->release(b.elig);
   c->release(b.loss);
   c->release(b.keys[0]); c->release(b.keys[1]); c->release(b.slots[0]); c->release(b.slots[1]);
-  c->release(b.ghist); c->release(b.G); c->release(b.ufeat); c->release(b.long_st); c->release(b.long_len);
+  c->release(b.ghist); c->release(b.dgrp); c->release(b.G); c->release(b.ufeat); c->release(b.long_st); c->release(b.long_len);
   c->release(b.long_pbase); c->release(b.long_runs); c->release(b.long_rlen); c->release(b.piece_st);
   c->release(b.piece_info);
   c->release(b.part); c->release(b.srec); c->release(b.mrec); c->release(b.scount); c->release(b.mcount);
