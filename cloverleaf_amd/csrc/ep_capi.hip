@@ -22,9 +22,10 @@
 // Step buffers of ep_step_explicit_noalloc: one array per GPU, held from the library's
 // load until the process ends.  Host code never uses this name as an address (on the
 // host it is a stand-in): the device address comes from hipGetSymbolAddress, once per
-// device (scratch_ptr).  Every call on a GPU shares that GPU's array.
+// device (scratch_ptr).  Every call on a GPU shares that GPU's array.  The sort's totals lie
+// after the step's arrays and don't count against their limit.
 constexpr size_t kScratchBytes = (size_t)64 << 20;
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+static __device__ __align__(256) unsigned char scratch[kScratchBytes + ep::kSortTotals * sizeof(uint32_t)];
 
 namespace {
 
@@ -367,10 +368,11 @@ uint64_t example_rows_max(const ep_ctx* c) {
   return (uint64_t)c->f_max * (1ull + neighbour_cap(c) + c->cfg.negatives);
 }
 
-// Places every per-step array of StepConfig b for batches of up to `batch` anchors and
-// sets the step's capacities and grid shapes.  place(&ptr, count) gives an array its
-// memory: hipMalloc (ensure_step_buffers) or a carve-out of the no-allocation scratch
-// (ep_step_explicit_noalloc).  *keycap_out receives the key capacity.
+// Places every per-step array of StepConfig b but the sort's totals (dgrp, of one size for
+// every step) for batches of up to `batch` anchors and sets the step's capacities and grid
+// shapes.  place(&ptr, count) gives an array its memory: hipMalloc (ensure_step_buffers) or a
+// carve-out of the no-allocation scratch (ep_step_explicit_noalloc).  *keycap_out receives the
+// key capacity.
 template <typename Place>
 int place_step_buffers(ep_ctx* c, uint32_t batch, ep::StepConfig& b, Place&& place, uint64_t* keycap_out) {
   const ep_config& cfg = c->cfg;
@@ -459,7 +461,6 @@ int place_step_buffers(ep_ctx* c, uint32_t batch, ep::StepConfig& b, Place&& pla
     EP_TRY(place(&b.slots[i], keycap));
   }
   EP_TRY(place(&b.ghist, (size_t)2048 * sort_grid));
-  EP_TRY(place(&b.dgrp, ep::kSortTotals));
   EP_TRY(place(&b.long_st, long_cap));
   EP_TRY(place(&b.long_len, long_cap));
   EP_TRY(place(&b.long_pbase, long_cap));
@@ -574,6 +575,7 @@ int ensure_step_buffers(ep_ctx* c, uint32_t batch) {
 
   uint64_t keycap = 0;
   EP_TRY(place_step_buffers(c, batch, b, [c](auto** p, size_t n) { return c->alloc(p, n); }, &keycap));
+  EP_TRY(c->alloc(&b.dgrp, ep::kSortTotals));
   const uint32_t P = std::max<uint32_t>(1u, cfg.concurrent_batches);
   // merged-gradient records (G, ufeat) only serve the test hook's gradient output (one per
   // (row, batch) run); they are allocated by ep_step_explicit on first use
@@ -1600,6 +1602,7 @@ int ep_step_explicit_noalloc(ep_ctx* c, const uint32_t* anchors, uint32_t n, con
   if (need > kScratchBytes)
     return fail(EP_ECAPACITY, "ep_step_explicit_noalloc: the step needs " + std::to_string(need) +
                                   " bytes of scratch, the library holds " + std::to_string(kScratchBytes));
+  sc.dgrp = reinterpret_cast<uint32_t*>(c->scratch + kScratchBytes);
   sc.perm = d_anchors;
   sc.negpool = d_anchors;
   sc.n_negpool = n;
