@@ -61,14 +61,16 @@ void shuffle(std::vector<T>& v, HostRng& r) {
   for (size_t i = v.size(); i > 1; --i) std::swap(v[i - 1], v[r.below(i)]);
 }
 
-// Copies device memory to a caller's (pageable) array after the work queued on the stream.  From
+// Copies device memory to a caller's array after the work queued on the stream.  From
 // kMinBytes up through a ring of pinned chunks: the copy engine fills chunks while a few
 // threads move filled ones out, taking the page faults of a fresh array side by side.  The
 // runtime's own pageable copy waits for the faults and the transfer in turn: 51 MB into a fresh
 // array take it 5.2 ms on a MI355X host and 3.0 into a touched one, the transfer alone 1.0;
-// this takes 1.6.  Starting the threads costs about what 10 MB gain: a call with 8.4 MB of
-// results took 0.2 ms longer this way, with 10 MB 0.1, with 15 MB 0.4 less.  The ring (8 MB) belongs to one context or aligner, from its first large
-// copy to its end; the threads end with the copy.
+// this takes 1.6.  An array that is page-locked itself is left to the runtime, which has the
+// engine write it.  Starting the threads costs about what 10 MB gain: a call with 8.4 MB of
+// results took 0.2 ms longer this way, with 10 MB 0.1, with 15 MB 0.4 less.  The ring (8 MB)
+// belongs to one context or aligner, from its first large copy to its end; the threads end
+// with the copy.
 class HostCopy {
  public:
   HostCopy() = default;
@@ -81,10 +83,11 @@ class HostCopy {
   }
 
   hipError_t run(void* dst, const void* src, size_t bytes, hipStream_t s) {
-    // a second thread reading from the same context meanwhile takes the runtime's copy
-    std::unique_lock<std::mutex> own(use_, std::try_to_lock);
-    if (bytes >= kMinBytes && own && prepare() && start()) return copy((unsigned char*)dst, (const unsigned char*)src, bytes, s);
-    if (own) own.unlock();
+    if (bytes >= kMinBytes && !page_locked(dst)) {
+      // a second thread reading from the same context meanwhile takes the runtime's copy
+      std::unique_lock<std::mutex> own(use_, std::try_to_lock);
+      if (own && prepare() && start()) return copy((unsigned char*)dst, (const unsigned char*)src, bytes, s);
+    }
     hipError_t e = bytes ? hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s) : hipSuccess;
     return e == hipSuccess ? hipStreamSynchronize(s) : e;
   }
@@ -92,6 +95,14 @@ class HostCopy {
  private:
   static constexpr size_t kMinBytes = (size_t)12 << 20, kChunk = (size_t)1 << 20;
   static constexpr int kRing = 8, kFlight = 3, kThreads = 6;  // chunks, copies in flight, threads
+
+  // Whether the runtime knows the caller's array as memory that the device can write.
+  static bool page_locked(const void* p) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+    return false;
+  }
 
   // The ring and its events; false when they are not to be had.
   bool prepare() {
