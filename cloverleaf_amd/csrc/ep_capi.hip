@@ -68,9 +68,13 @@ void shuffle(std::vector<T>& v, HostRng& r) {
 // array take it 5.2 ms on a MI355X host and 3.0 into a touched one, the transfer alone 1.0;
 // this takes 1.6.  An array that is page-locked itself is left to the runtime, which has the
 // engine write it.  Starting the threads costs about what 10 MB gain: a call with 8.4 MB of
-// results took 0.2 ms longer this way, with 10 MB 0.1, with 15 MB 0.4 less.  The ring (8 MB)
-// belongs to one context or aligner, from its first large copy to its end; the threads end
-// with the copy.
+// results took 0.2 ms longer this way, with 10 MB 0.1, with 15 MB 0.4 less.
+//
+// Rows that the device holds in another layout (run_rows) are written into the chunks by a
+// kernel instead, at any size: no device memory to stage them in.
+//
+// The ring (8 MB, 2 while only smaller reads of rows used it) belongs to one context or aligner,
+// from its first such copy to its end; the threads end with the copy.
 class HostCopy {
  public:
   HostCopy() = default;
@@ -86,15 +90,36 @@ class HostCopy {
     if (bytes >= kMinBytes && !page_locked(dst)) {
       // a second thread reading from the same context meanwhile takes the runtime's copy
       std::unique_lock<std::mutex> own(use_, std::try_to_lock);
-      if (own && prepare() && start()) return copy((unsigned char*)dst, (const unsigned char*)src, bytes, s);
+      if (own && prepare(kRing) && start())
+        return copy(dst, bytes, kChunk, s, [&](size_t at, size_t n, unsigned char* to) {
+          return hipMemcpyAsync(to, (const unsigned char*)src + at, n, hipMemcpyDeviceToHost, s);
+        });
     }
     hipError_t e = bytes ? hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s) : hipSuccess;
     return e == hipSuccess ? hipStreamSynchronize(s) : e;
   }
 
+  // rows rows of row_bytes (at most kChunk) each: fill(first, count, to) queues the kernel that
+  // writes rows [first, first + count) to `to`.  *done is false when there was no pinned
+  // memory (nothing was copied then).  A second thread waits for its turn.
+  template <typename Fill>
+  hipError_t run_rows(void* dst, size_t rows, size_t row_bytes, hipStream_t s, bool* done, Fill fill) {
+    const size_t per = kChunk / row_bytes, bytes = rows * row_bytes;
+    std::lock_guard<std::mutex> own(use_);
+    const bool small = bytes < kMinBytes;
+    *done = prepare((int)std::min<size_t>(small ? kSmallRing : kRing, (rows + per - 1) / per));
+    if (!*done) return hipSuccess;
+    if (!small) (void)start();  // small reads, and others with no threads to be had: copy() moves the chunks out
+    return copy(dst, bytes, per * row_bytes, s, [&](size_t at, size_t n, unsigned char* to) {
+      return fill(at / row_bytes, n / row_bytes, (float*)(dev_ring_ + (to - ring_)));
+    });
+  }
+
  private:
   static constexpr size_t kMinBytes = (size_t)12 << 20, kChunk = (size_t)1 << 20;
-  static constexpr int kRing = 8, kFlight = 3, kThreads = 6;  // chunks, copies in flight, threads
+  // chunks, chunks where one thread empties them (the first touch of pinned memory takes it
+  // 0.35 ms a chunk on a MI355X host), copies in flight, threads
+  static constexpr int kRing = 8, kSmallRing = 2, kFlight = 3, kThreads = 6;
 
   // Whether the runtime knows the caller's array as memory that the device can write.
   static bool page_locked(const void* p) {
@@ -104,27 +129,29 @@ class HostCopy {
     return false;
   }
 
-  // The ring and its events; false when they are not to be had.
-  bool prepare() {
-    if (!ring_ && hipHostMalloc((void**)&ring_, kRing * kChunk, hipHostMallocDefault) != hipSuccess) {
-      ring_ = nullptr;
-      (void)hipGetLastError();
-      return false;
+  // The ring, of at least this many chunks, and its events; false when they are not to be had.
+  bool prepare(int chunks) {
+    hipError_t e = hipSuccess;
+    if (parts_ < (size_t)chunks) {
+      if (ring_) (void)hipHostFree(ring_);
+      ring_ = dev_ring_ = nullptr;
+      parts_ = 0;
+      e = hipHostMalloc((void**)&ring_, chunks * kChunk, hipHostMallocCoherent);  // kernels write it too
+      if (e != hipSuccess) ring_ = nullptr;
+      else e = hipHostGetDevicePointer((void**)&dev_ring_, ring_, 0);
+      if (e == hipSuccess) parts_ = chunks;
     }
-    for (hipEvent_t& e : ev_)
-      if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-        e = nullptr;
-        (void)hipGetLastError();
-        return false;
+    for (int i = 0; i < kRing && e == hipSuccess; ++i)
+      if (!ev_[i]) {
+        e = hipEventCreateWithFlags(&ev_[i], hipEventDisableTiming);
+        if (e != hipSuccess) ev_[i] = nullptr;
       }
-    return true;
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e == hipSuccess;
   }
 
   // The threads of a copy: as many as there are to be had, false for none.
   bool start() {
-    ready_ = taken_ = 0;
-    last_ = false;
-    for (size_t& n : out_) n = 0;
     try {
       for (std::thread& t : threads_) t = std::thread([this] { work(); });
     } catch (...) {
@@ -132,31 +159,38 @@ class HostCopy {
     return threads_[0].joinable();
   }
 
-  hipError_t copy(unsigned char* dst, const unsigned char* src, size_t bytes, hipStream_t s) {
-    dst_ = dst;
+  // Copies bytes in chunks of step: fill(at, n, to) queues the copy of bytes [at, at + n).
+  template <typename Fill>
+  hipError_t copy(void* dst, size_t bytes, size_t step, hipStream_t s, Fill fill) {
+    dst_ = (unsigned char*)dst;
     bytes_ = bytes;
-    const size_t n = (bytes + kChunk - 1) / kChunk;
+    step_ = step;
+    const bool alone = !threads_[0].joinable();
+    const size_t n = (bytes + step - 1) / step, flight = std::min<size_t>(kFlight, parts_ - 1);
     hipError_t e = hipSuccess;
-    for (size_t c = 0; c < n + kFlight && e == hipSuccess; ++c) {
+    for (size_t c = 0; c < n + flight && e == hipSuccess; ++c) {
       if (c < n) {
-        if (c >= (size_t)kRing) {  // the chunk that used this part of the ring has left it
+        if (c >= parts_) {  // the chunk that used this part of the ring has left it
           std::unique_lock<std::mutex> lk(mu_);
-          cv_.wait(lk, [&] { return out_[c % kRing] > (c - kRing) / kRing; });
+          cv_.wait(lk, [&] { return out_[c % parts_] > (c - parts_) / parts_; });
         }
-        e = hipMemcpyAsync(ring_ + c % kRing * kChunk, src + c * kChunk, std::min(kChunk, bytes - c * kChunk),
-                           hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipEventRecord(ev_[c % kRing], s);
+        e = fill(c * step, std::min(step, bytes - c * step), ring_ + c % parts_ * kChunk);
+        if (e == hipSuccess) e = hipEventRecord(ev_[c % parts_], s);
       }
-      if (e == hipSuccess && c >= (size_t)kFlight) {
-        e = hipEventSynchronize(ev_[(c - kFlight) % kRing]);
-        if (e == hipSuccess) {
+      if (e == hipSuccess && c >= flight) {
+        const size_t r = c - flight;
+        e = hipEventSynchronize(ev_[r % parts_]);
+        if (e == hipSuccess && alone) {
+          move_out(r);
+          ++out_[r % parts_];
+        } else if (e == hipSuccess) {
           std::lock_guard<std::mutex> lk(mu_);
-          ready_ = c - kFlight + 1;
+          ready_ = r + 1;
         }
         cv_.notify_all();
       }
     }
-    if (e != hipSuccess) (void)hipStreamSynchronize(s);  // no copy into the ring may be left
+    if (e != hipSuccess) (void)hipStreamSynchronize(s);  // nothing may be left that writes into the ring
     stop(e != hipSuccess);
     return e;
   }
@@ -171,6 +205,13 @@ class HostCopy {
     cv_.notify_all();
     for (std::thread& t : threads_)
       if (t.joinable()) t.join();
+    ready_ = taken_ = 0;
+    last_ = false;
+    for (size_t& x : out_) x = 0;
+  }
+
+  void move_out(size_t c) {
+    std::memcpy(dst_ + c * step_, ring_ + c % parts_ * kChunk, std::min(step_, bytes_ - c * step_));
   }
 
   void work() {
@@ -180,21 +221,23 @@ class HostCopy {
       if (taken_ >= ready_) return;
       const size_t c = taken_++;
       lk.unlock();
-      std::memcpy(dst_ + c * kChunk, ring_ + c % kRing * kChunk, std::min(kChunk, bytes_ - c * kChunk));
+      move_out(c);
       lk.lock();
-      ++out_[c % kRing];
+      ++out_[c % parts_];
       cv_.notify_all();
     }
   }
 
   unsigned char* ring_ = nullptr;
+  unsigned char* dev_ring_ = nullptr;  // the device's address of the ring
+  size_t parts_ = 0;                   // chunks in the ring
   hipEvent_t ev_[kRing] = {};
   std::thread threads_[kThreads];
   std::mutex use_;  // the ring and the threads, for one copy
   std::mutex mu_;
   std::condition_variable cv_;
   unsigned char* dst_ = nullptr;
-  size_t bytes_ = 0;
+  size_t bytes_ = 0, step_ = 0;
   size_t ready_ = 0, taken_ = 0;  // chunks filled, chunks given to a thread
   size_t out_[kRing] = {};        // chunks moved out of each part of the ring
   bool last_ = false;             // no more chunks will come
@@ -1189,48 +1232,30 @@ int ep_set_table(ep_ctx* c, const float* rows) {
   return EP_OK;
 }
 
-// Copies a rows x D FP32 array that the device holds in another layout: stage(first, count,
-// dst) fills dst with rows [first, first + count) on the context's stream, at most 64 MiB of
-// them at a time (halved while that cannot be allocated), each chunk copied out in one piece.
-// *staged is false when no device memory was left to stage in (nothing was copied then).
-extern "C++" template <typename Stage>
-static int copy_staged(ep_ctx* c, float* out, uint64_t rows, uint32_t D, bool* staged, Stage stage) {
-  const uint64_t row_bytes = (uint64_t)D * sizeof(float);
-  uint64_t chunk = std::min<uint64_t>(rows, std::max<uint64_t>(((uint64_t)64 << 20) / row_bytes, 1));
-  float* buf = nullptr;
-  *staged = false;
-  while (hipMalloc((void**)&buf, chunk * row_bytes) != hipSuccess) {
-    (void)hipGetLastError();
-    if (chunk == 1) return EP_OK;
-    chunk = (chunk + 1) / 2;
-  }
-  *staged = true;
-  hipError_t e = hipSuccess;
-  for (uint64_t r = 0; r < rows && e == hipSuccess; r += chunk) {
-    const uint64_t n = std::min(chunk, rows - r);
-    e = stage(r, n, buf);
-    if (e == hipSuccess) e = c->to_host.run(out + r * D, buf, n * row_bytes, c->stream);
-  }
-  (void)hipFree(buf);
-  if (e != hipSuccess) return fail(EP_EHIP, std::string("staged copy: ") + hipGetErrorString(e));
+// The table's rows to out[n_vocab * D], written by fill's kernel (HostCopy::run_rows).
+extern "C++" template <typename Fill>
+static int copy_rows(ep_ctx* c, float* out, uint32_t D, bool* done, Fill fill) {
+  const hipError_t e = c->to_host.run_rows(out, c->n_vocab, D * sizeof(float), c->stream, done, fill);
+  if (e != hipSuccess) return fail(EP_EHIP, std::string("copy of rows: ") + hipGetErrorString(e));
   return EP_OK;
 }
 
-// One D-wide part of the optimizer records (master, m or v) to out[n_vocab * D]: packed on the
-// device first (a pitched copy moves row by row), pitched only when there is no memory left.
+// One D-wide part of the optimizer records (master, m or v) to out[n_vocab * D]: packed by a
+// kernel on its way (a pitched copy moves row by row), pitched where there is no pinned memory.
 static int copy_record_part(ep_ctx* c, const float* part, uint32_t D, uint32_t ostride, float* out) {
-  bool staged = false;
-  EP_TRY(copy_staged(c, out, c->n_vocab, D, &staged, [&](uint64_t r, uint64_t n, float* dst) {
-    return ep::launch_pack_rows(part + r * ostride, dst, n, D, ostride, c->stream);
+  bool done = false;
+  EP_TRY(copy_rows(c, out, D, &done, [&](uint64_t r, uint64_t n, float* to) {
+    return ep::launch_pack_rows(part + r * ostride, to, n, D, ostride, c->stream);
   }));
-  if (!staged)
+  if (!done)
     EP_HIP(hipMemcpy2D(out, D * sizeof(float), part, ostride * sizeof(float), D * sizeof(float), c->n_vocab,
                        hipMemcpyDeviceToHost));
   return EP_OK;
 }
 
-// MI355X host: 8.4M values take 3.3 ms either way, 25.6M 9.9 ms against 18.6 on the host, 4.2M
-// 1.1 ms against 0.84.
+// MI355X host, a read into a fresh array, first of its context / later: 8.4M values 2.3 / 1.2 ms
+// this way against 3.4 / 3.2 widened on the host, 25.6M 4.4 / 3.4 against 19.7 / 19.2; 4.2M take
+// 3.4 / 0.9 on the host.
 constexpr size_t kWidenOnDevice = (size_t)1 << 23;
 
 int ep_get_table(ep_ctx* c, float* rows) {
@@ -1243,14 +1268,13 @@ int ep_get_table(ep_ctx* c, float* rows) {
   const size_t n = (size_t)c->n_vocab * D;
   if (c->cfg.precision == EP_PREC_BF16) {
     // the bf16 table is the parameter, widened (exact) on the device from kWidenOnDevice
-    // values up; smaller tables, where the staging buffer's allocation costs more than the
-    // widening, and tables with no memory left to stage in, here
-    bool staged = false;
+    // values up; smaller tables, and tables with no pinned memory to be had, here
+    bool done = false;
     if (n >= kWidenOnDevice)
-      EP_TRY(copy_staged(c, rows, c->n_vocab, D, &staged, [&](uint64_t r, uint64_t k, float* dst) {
-        return ep::launch_widen_bf16((const uint16_t*)c->d_table + r * D, dst, k * D, c->stream);
+      EP_TRY(copy_rows(c, rows, D, &done, [&](uint64_t r, uint64_t k, float* to) {
+        return ep::launch_widen_bf16((const uint16_t*)c->d_table + r * D, to, k * D, c->stream);
       }));
-    if (staged) return EP_OK;
+    if (done) return EP_OK;
     std::vector<uint16_t> h(n);
     EP_HIP(hipMemcpy(h.data(), c->d_table, n * sizeof(uint16_t), hipMemcpyDeviceToHost));
     for (size_t i = 0; i < n; ++i) {

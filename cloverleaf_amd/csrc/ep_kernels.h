@@ -290,7 +290,7 @@ hipError_t launch_adam_touched(const StepConfig& c, StepState* st, hipStream_t s
 hipError_t launch_init_table(const StepConfig& c, uint64_t seed, hipStream_t s);
 hipError_t launch_fill_bf16(const float* src, uint16_t* dst, uint64_t n, uint32_t D, uint32_t stride, hipStream_t s);
 // Rows of a strided record array packed (D and stride multiples of 4), BF16 values widened
-// (n a multiple of 4): what the table and moment reads stage for the copy to the host.
+// (n a multiple of 4): the table and moment reads, dst pinned host memory.
 hipError_t launch_pack_rows(const float* src, float* dst, uint64_t rows, uint32_t D, uint32_t stride, hipStream_t s);
 hipError_t launch_widen_bf16(const uint16_t* src, float* dst, uint64_t n, hipStream_t s);
 hipError_t launch_embed_averaged(const StepConfig& c, const uint64_t* findptr, const uint32_t* fids,

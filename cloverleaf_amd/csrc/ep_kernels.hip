@@ -3092,9 +3092,9 @@ __global__ void k_fill_bf16(const float* __restrict__ src, uint16_t* __restrict_
 }
 
 // dst[r*D4 + j] = src[r*stride4 + j] in 16-byte columns for rows r < rows: one part (master,
-// m or v) of the optimizer records packed for the copy to the host.  Bound by the copy that
-// follows; a pitched device-to-host copy moves row by row (7 us per 1 KB row on MI355X,
-// 820 ms for 120k rows of 256 values), packed rows leave at the speed of a plain copy.
+// m or v) of the optimizer records packed into pinned host memory.  Bound by the link to the
+// host; a pitched device-to-host copy moves row by row (7 us per 1 KB row on MI355X, 820 ms for
+// 120k rows of 256 values).
 __global__ __launch_bounds__(256) void k_pack_rows(const float4* __restrict__ src, float4* __restrict__ dst,
                                                    uint64_t rows, uint32_t D4, uint32_t stride4) {
   const uint64_t n = rows * D4, step = (uint64_t)gridDim.x * blockDim.x;
@@ -3542,12 +3542,16 @@ hipError_t launch_fill_bf16(const float* src, uint16_t* dst, uint64_t n, uint32_
 }
 
 hipError_t launch_pack_rows(const float* src, float* dst, uint64_t rows, uint32_t D, uint32_t stride, hipStream_t s) {
-  hipLaunchKernelGGL(k_pack_rows, dim3(2048), dim3(256), 0, s, (const float4*)src, (float4*)dst, rows, D / 4, stride / 4);
+  const uint64_t blocks = (rows * (D / 4) + 255u) / 256u;
+  hipLaunchKernelGGL(k_pack_rows, dim3((uint32_t)std::min<uint64_t>(blocks, 2048)), dim3(256), 0, s, (const float4*)src,
+                     (float4*)dst, rows, D / 4, stride / 4);
   return hipGetLastError();
 }
 
 hipError_t launch_widen_bf16(const uint16_t* src, float* dst, uint64_t n, hipStream_t s) {
-  hipLaunchKernelGGL(k_widen_bf16, dim3(2048), dim3(256), 0, s, (const uint2*)src, (float4*)dst, n / 4);
+  const uint64_t blocks = (n / 4 + 255u) / 256u;
+  hipLaunchKernelGGL(k_widen_bf16, dim3((uint32_t)std::min<uint64_t>(blocks, 2048)), dim3(256), 0, s, (const uint2*)src,
+                     (float4*)dst, n / 4);
   return hipGetLastError();
 }
 
