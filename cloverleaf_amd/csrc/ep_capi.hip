@@ -322,15 +322,17 @@ struct ep_ctx {
   hipGraphExec_t step_exec = nullptr;
   bool step_exec_ready = false;
 
-  // segment-Adam variant tuner: the first training steps rotate through the supported
-  // values-per-lane variants (identical results) and time the scatter with events
-  int seg_vpl = 0;                 // chosen variant (values per lane, unroll), 0 while tuning
+  // variant tuner: the first training steps rotate through the supported segment tiles and
+  // k_forward variants (identical results) and time them with events
+  int seg_vpl = 0;                 // chosen tile (values per lane, unroll), 0 while not chosen
   int seg_unroll = 0;
-  int fwd_x = 0;                   // chosen k_forward variant (rows-in-flight multiplier), 0 while tuning
+  int fwd_x = 0;                   // chosen k_forward variant (rows-in-flight multiplier), 0 while not chosen
   std::vector<std::pair<int, int>> tune_cands;
   std::vector<int> tune_fwd;       // k_forward candidates, timed in the same steps
-  std::vector<hipEvent_t> tune_ev;  // two per tuning step
+  std::vector<hipEvent_t> tune_ev;  // nine per tuning step
   uint32_t tune_i = 0;
+  bool tune_one = false;           // the tuning steps take one row launch
+  bool tuned_one = false;          // k_forward has been tuned over such steps (the tile has not)
 
   ~ep_ctx() {
     for (hipEvent_t e : tune_ev) (void)hipEventDestroy(e);
@@ -728,6 +730,7 @@ void refresh_base(ep_ctx* c) {
   b.seed = cfg.seed;
   b.alpha = cfg.alpha;
   b.scatter = cfg.scatter;
+  b.any_tile = cfg.seg_vpl == 0 ? 1 : 0;
   b.train = 1;
   b.explicit_samples = 0;
   b.pass_loss = nullptr;
@@ -746,7 +749,6 @@ void refresh_base(ep_ctx* c) {
 void pick_variant(const ep_ctx* c, ep::StepConfig& sc) {
   if (sc.fwd_x == 0) sc.fwd_x = c->fwd_x ? c->fwd_x : 1;
   if (sc.seg_vpl != 0) return;  // the tuner's candidate
-  sc.any_tile = c->cfg.seg_vpl == 0 ? 1 : 0;
   sc.seg_vpl = c->seg_vpl ? c->seg_vpl : 4;
   sc.seg_unroll = c->seg_vpl ? c->seg_unroll : 8;
 }
@@ -874,21 +876,50 @@ ep::StepConfig train_config(ep_ctx* c) {
 // Number of tuning rounds; the first round is a warm-up and is not scored.
 constexpr uint32_t kTuneRounds = 4;
 
-bool tuning(const ep_ctx* c) { return c->cfg.scatter == EP_SCATTER_SORT && c->seg_vpl == 0; }
+// Whether the step's rows take k_rows, whose tile is fixed.
+bool one_row_launch(const ep_ctx* c) {
+  return c->cfg.scatter == EP_SCATTER_SORT && ep::rows_in_one_launch(c->base);
+}
+
+bool tuning(const ep_ctx* c) {
+  return c->cfg.scatter == EP_SCATTER_SORT && c->seg_vpl == 0 && !(c->tuned_one && one_row_launch(c));
+}
+
+void clear_tuner(ep_ctx* c) {
+  for (hipEvent_t e : c->tune_ev) (void)hipEventDestroy(e);
+  c->tune_ev.clear();
+  c->tune_cands.clear();
+  c->tune_fwd.clear();
+  c->tune_i = 0;
+}
 
 // One eager training step with the next candidate variants; after the last tuning step
 // the fastest variant of each kernel (median time over the scored rounds) is fixed.  The
 // k_seg_update candidates rotate with the step index modulo their count, the k_forward
-// candidates modulo theirs; a round is as many steps as the larger count.
+// candidates modulo theirs; a round is as many steps as the larger count.  Steps with one
+// row launch have no tile to choose: k_forward's variants are timed in that route, over as
+// many steps, and a context whose later steps are too large for it tunes the tile then.
 int tune_step(ep_ctx* c, const ep::StepConfig& sc) {
+  const bool one = one_row_launch(c);
+  if (!c->tune_cands.empty() && c->tune_one != one) clear_tuner(c);
+  auto choose = [&](std::pair<int, int> tile, int fwd) {
+    if (one) {
+      c->tuned_one = true;
+    } else {
+      c->seg_vpl = tile.first;
+      c->seg_unroll = tile.second;
+    }
+    c->fwd_x = fwd;
+    clear_tuner(c);
+  };
   if (c->tune_cands.empty()) {
+    c->tune_one = one;
     for (int v : {16, 12, 8, 4})
       for (int u : {v == 12 ? 2 : 8 / (v / 4), v == 12 ? 4 : 16 / (v / 4)})
         if (ep::seg_variant_supported((int)row_width(c->cfg), v, u)) c->tune_cands.push_back({v, u});
     if (c->tune_cands.empty()) c->tune_cands.push_back({4, 8});
-    c->tune_fwd.clear();
-    if (c->cfg.forward_variant) {
-      c->tune_fwd.push_back(c->cfg.forward_variant);
+    if (c->fwd_x) {
+      c->tune_fwd.push_back(c->fwd_x);
     } else {
       for (int x : {1, 2})
         if (!c->cfg.attention_dk && ep::fwd_variant_supported((int)row_width(c->cfg), c->cfg.precision != EP_PREC_FP32, x))
@@ -896,9 +927,7 @@ int tune_step(ep_ctx* c, const ep::StepConfig& sc) {
     }
     if (c->tune_fwd.empty()) c->tune_fwd.push_back(1);
     if (c->tune_cands.size() <= 1 && c->tune_fwd.size() <= 1) {
-      c->seg_vpl = c->tune_cands[0].first;
-      c->seg_unroll = c->tune_cands[0].second;
-      c->fwd_x = c->tune_fwd[0];
+      choose(c->tune_cands[0], c->tune_fwd[0]);
       return launch_training_step(c, sc, true, -1.f);
     }
     const size_t ne = 9 * std::max(c->tune_cands.size(), c->tune_fwd.size()) * kTuneRounds;
@@ -909,8 +938,11 @@ int tune_step(ep_ctx* c, const ep::StepConfig& sc) {
   const uint32_t per_round = std::max(n, nf);
   const uint32_t i = c->tune_i++;
   ep::StepConfig t = sc;
-  t.seg_vpl = c->tune_cands[i % n].first;
-  t.seg_unroll = c->tune_cands[i % n].second;
+  if (!one) {
+    t.any_tile = 0;
+    t.seg_vpl = c->tune_cands[i % n].first;
+    t.seg_unroll = c->tune_cands[i % n].second;
+  }
   t.fwd_x = c->tune_fwd[i % nf];
   hipEvent_t evs[9];
   for (int k = 0; k < 9; ++k) evs[k] = c->tune_ev[9 * i + k];
@@ -944,9 +976,7 @@ int tune_step(ep_ctx* c, const ep::StepConfig& sc) {
     EP_TRY(median(nf, k, 1, 2, &med));  // forward
     if (med < bestf) { bestf = med; pickf = c->tune_fwd[k]; }
   }
-  c->seg_vpl = pick.first;
-  c->seg_unroll = pick.second;
-  c->fwd_x = pickf;
+  choose(pick, pickf);
   return EP_OK;
 }
 
@@ -1741,8 +1771,9 @@ int ep_bench_steps(ep_ctx* c, uint32_t warmup, uint32_t steps, int instrument, e
   out->unique_rows = h1.rows - h0.rows;
   out->att_items_sq = h1.stat_att_n2 - h0.stat_att_n2;
   out->att_items = h1.stat_att_n - h0.stat_att_n;
-  out->seg_vpl = c->seg_vpl;
-  out->seg_unroll = c->seg_unroll;
+  const bool one = one_row_launch(c);
+  out->seg_vpl = one ? ep::kRowsVpl : c->seg_vpl;
+  out->seg_unroll = one ? ep::kRowsUnroll : c->seg_unroll;
   out->fwd_x = c->fwd_x ? c->fwd_x : 1;
   if (instrument) {
     // per-phase timing: the same number of steps launched one by one with events

@@ -230,9 +230,9 @@ struct StepConfig {
   int grad_out;            // test hook: write merged gradients (G/ufeat) instead of updating;
                            // ufeat = row | batch << 27
   int unique_grid;         // grid size for the persistent row kernels
-  int seg_vpl;             // k_seg_adam values per lane (4, 8, 16; chosen by the tuner)
+  int seg_vpl;             // k_seg_update values per lane (4, 8, 12, 16; chosen by the tuner)
   int any_tile;            // 1: the tile was not asked for by name and is not being tuned
-  int seg_unroll;          // k_seg_adam adjoint rows in flight per lane group (tuned)
+  int seg_unroll;          // k_seg_update adjoint rows in flight per lane group (tuned)
   int fwd_x;               // k_forward rows-in-flight multiplier of the wide gathers: 1 or 2 (tuned)
   // Attention model (model = 1): rows are [Q_1..Q_H | K_1..K_H | V_1..V_H], dims =
   // att_heads * (2 att_dk + att_dm).  An example's attention blocks (h(v), one per
@@ -320,7 +320,11 @@ hipError_t launch_att_embed(const StepConfig& c, const uint64_t* findptr, const 
 constexpr uint32_t kSegShort = 32;
 constexpr uint32_t kPieceEntries = 32;
 bool seg_vpl_supported(int d, int vpl);
-// Whether k_seg_adam<D, VPL, U> is built (U in {8, 16} / (VPL/4)).
+// Whether the step's short and medium rows and pieces take one launch (k_rows), and the segment
+// tile of its short rows.
+bool rows_in_one_launch(const StepConfig& c);
+constexpr int kRowsVpl = 4, kRowsUnroll = 8;
+// Whether k_seg_update<D, VPL, U> is built (U in {8, 16} / (VPL/4)).
 bool seg_variant_supported(int d, int vpl, int unroll);
 // Forward variants: x = 1, and x = 2 (twice the rows in flight) where the wide gather runs.
 bool fwd_variant_supported(int d, int bf16, int x);

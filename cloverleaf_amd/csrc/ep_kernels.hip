@@ -2880,10 +2880,6 @@ __global__ __launch_bounds__(256) void k_pieces(StepConfig c, StepState* st, con
   medium_rows<D, H>(c, st, Ks, Ss, blockIdx.x, gridDim.x);
 }
 
-// The segment tile of a launch that has no tuned one.
-template <int D> constexpr int kTileV = (D % 4 == 0 && D / 4 <= 64) ? 4 : 16;
-template <int D> constexpr int kTileU = kTileV<D> == 4 ? 8 : 2;
-
 // Small steps: the pieces, the medium rows and the short rows are different rows, so blocks
 // of one launch take them side by side; one after the other each is a chain of loads on a device
 // mostly idle (see rows_in_one_launch for both times).
@@ -2893,7 +2889,7 @@ __global__ __launch_bounds__(256) void k_rows(StepConfig c, StepState* st, const
   const uint32_t b = blockIdx.x;
   if (b < nmed) medium_rows<D, H>(c, st, Ks, Ss, b, nmed);
   else if (b < nmed + npiece) piece_sums<D, H>(c, st, Ss, b - nmed, npiece);
-  else short_rows<D, kTileV<D>, kTileU<D>, H, false>(c, st, Ss, b - nmed - npiece, gridDim.x - nmed - npiece);
+  else short_rows<D, kRowsVpl, kRowsUnroll, H, false>(c, st, Ss, b - nmed - npiece, gridDim.x - nmed - npiece);
 }
 
 // One wave per long row: loads theta/m/v once, adds the pieces of each run in order and
@@ -3433,7 +3429,7 @@ bool seg_variant_supported(int d, int vpl, int unroll) {
 // MI355X, one launch against two: 16k keys of D = 64 11.8 against 21.2 us, 0.4M keys of
 // D = 128 45 against 60; at D = 768 (256 VGPRs, one wave per SIMD for every role) it gains
 // nothing, so the attention widths past 256 keep two.
-static bool rows_in_one_launch(const StepConfig& c) {
+bool rows_in_one_launch(const StepConfig& c) {
   return c.any_tile && c.dims <= 256 && c.key_cap <= kRowsOneLaunch && !(c.noise > 1e-9f);
 }
 
