@@ -63,6 +63,16 @@ def update_bytes(urows, dims, bytes_per_value, master=False):
     return urows * dims * ((bytes_per_value + 24) if master else (2 * bytes_per_value + 16))
 
 
+def update_figures(r, dims, bytes_per_value, master=False):
+    """Kernel name, bytes per step and ms of the row update.  Short rows have a kernel and a
+    phase of their own; where a step's rows take one launch (its other phase is exactly 0)
+    the figures are those of all rows, over that launch and the long rows' kernel."""
+    ph, one = r.ms_phase, r.ms_phase[5] > 0 and r.ms_phase[6] == 0
+    name, rows, ms = ("k_rows + k_long_combine", r.unique_rows, ph[5] + ph[7]) if one else \
+                     ("k_seg_update", r.short_rows, ph[5])
+    return name, update_bytes(rows, dims, bytes_per_value, master) / max(r.steps, 1), ms
+
+
 def attention_flops(att_items_sq, att_items, heads, dk, dm):
     """Attention FLOP model over the timed steps: per block of n items and per head,
     forward 2 n^2 d_k (scores) + n^2 (softmax) + 2 n d_model (weighted values); the
@@ -104,7 +114,7 @@ def run_form(w, form, steps, warmup, scatter=None, concurrent=1, graph=True, fp1
     ph = [float(x) for x in r.ms_phase]
     W = N.row_width(cfg)  # table row width (attention rows hold Q, K and V of every head)
     g_launch = gather_bytes(r.rows, r.nodes, r.examples, W, b) / S
-    u_launch = update_bytes(r.short_rows, W, b, prec == "bf16-master") / S
+    u_kernel, u_launch, u_ms = update_figures(r, W, b, prec == "bf16-master")
     step_bytes = (gather_bytes(r.rows, r.nodes, r.examples, W, b)
                   + update_bytes(r.unique_rows, W, b, prec == "bf16-master")) / S
     extra = {}
@@ -139,7 +149,9 @@ def run_form(w, form, steps, warmup, scatter=None, concurrent=1, graph=True, fp1
         "forward_bytes_per_launch": g_launch,
         "forward_gbs": g_launch / (ph[1] / 1e3) / 1e9 if ph[1] > 0 else 0.0,
         "update_bytes_per_launch": u_launch,
-        "update_gbs": u_launch / (ph[5] / 1e3) / 1e9 if ph[5] > 0 else 0.0,
+        "update_kernel": u_kernel,
+        "update_ms": round(u_ms, 4),
+        "update_gbs": u_launch / (u_ms / 1e3) / 1e9 if u_ms > 0 else 0.0,
         "step_bytes": step_bytes,
         "step_gbs": step_bytes / (r.ms_total / S / 1e3) / 1e9,
         **extra,
@@ -351,7 +363,7 @@ def main():
     cpu = None if args.no_cpu else cpu_baseline(w, args.cpu_budget)
     ph = head["phase_ms"]
     roof = None
-    if w.att_dk and ph["forward"] >= ph["short_update"]:
+    if w.att_dk and ph["forward"] >= head["update_ms"]:
         # the attention forward + backward (scores, softmax, weighted values, their
         # adjoints) on matrix cores and vector ALUs, against the FP32 dense peak
         tf = head["attention_tflops"]
@@ -362,10 +374,11 @@ def main():
                 "achieved": round(tf, 2), "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
                 "frac": round(tf / FP32_PEAK_TFLOPS, 4), "traffic": None,
                 "algorithmic_flops_per_launch": round(head["attention_flops_per_step"])}
-    if ph["short_update"] >= ph["forward"]:
-        kname, kdesc, kbytes, kgbs = ("k_seg_update", "short-row update: reduce runs of adjoint rows + Adam "
-                                      "(theta/m/v read and written once per row)",
-                                      head["update_bytes_per_launch"], head["update_gbs"])
+    if head["update_ms"] >= ph["forward"]:
+        kname = head["update_kernel"]
+        kdesc, kbytes, kgbs = (("short-row update" if kname == "k_seg_update" else "row update") +
+                               ": reduce runs of adjoint rows + Adam (theta/m/v read and written once per row)",
+                               head["update_bytes_per_launch"], head["update_gbs"])
     else:
         kname, kdesc, kbytes, kgbs = ("k_forward", "gather + mean + margin loss + adjoint",
                                       head["forward_bytes_per_launch"], head["forward_gbs"])

@@ -1796,6 +1796,7 @@ int ep_bench_steps(ep_ctx* c, uint32_t warmup, uint32_t steps, int instrument, e
         ph[k] += x;
       }
     for (auto& e : ev) (void)hipEventDestroy(e);
+    if (one) ph[6] = 0;  // k_rows has no time of its own for them
     for (int k = 0; k < 8; ++k) out->ms_phase[k] = ph[k] / steps;
     out->ms_forward_avg = out->ms_phase[1];
     out->ms_scatter_avg = out->ms_phase[3] + out->ms_phase[4] + out->ms_phase[5] + out->ms_phase[6] + out->ms_phase[7];

@@ -156,7 +156,10 @@ typedef struct ep_bench_result {
   int32_t seg_unroll;
   /* instrumented run: average duration per step of each phase, in ms:             */
   /* 0 step begin + sample + scan, 1 forward, 2 key emission, 3 radix sort,        */
-  /* 4 row plan, 5 short-row update, 6 pieces + medium rows, 7 long rows           */
+  /* 4 row plan, 5 short-row update, 6 pieces + medium rows, 7 long rows.  Steps of  */
+  /* at most 2^21 keys take phases 5 and 6 in one launch (unless the tile is named,  */
+  /* with noise, or past a row width of 256): its time is phase 5's, phase 6 is 0.   */
+  /* A phase that another one's kernel covers (scan, key emission) is near 0.        */
   double ms_phase[8];
   uint64_t short_rows;         /* rows updated by the short-row kernel (timed run)  */
   uint32_t last_long_rows;     /* long rows and their pieces in the last step        */

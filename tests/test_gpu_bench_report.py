@@ -1,4 +1,4 @@
-"""What ep_bench_steps reports about the row kernels: the segment tile in use."""
+"""What ep_bench_steps reports about the row kernels: the segment tile in use and the phases."""
 import numpy as np
 import pytest
 
@@ -33,6 +33,19 @@ def test_tile_of_small_steps(dims, prec):
 def test_tile_asked_for_by_name():
     r = bench(64, tile=(8, 4))
     assert (r.seg_vpl, r.seg_unroll) == (8, 4)
+
+
+def test_phases_of_one_launch():
+    """Short rows, medium rows and pieces in one launch: its time is the short rows' phase."""
+    r = bench(64)
+    assert r.ms_phase[5] > 0 and r.ms_phase[6] == 0 and r.ms_phase[7] > 0
+    assert r.ms_scatter_avg == pytest.approx(sum(r.ms_phase[3:8]))
+
+
+@pytest.mark.parametrize("kw", [dict(tile=(8, 4)), dict(noise=0.1), dict(batch=40_000)])
+def test_phases_of_separate_kernels(kw):
+    r = bench(64, **kw)
+    assert r.ms_phase[5] > 0 and r.ms_phase[6] > 0 and r.ms_phase[7] > 0
 
 
 def test_a_context_that_grows_tunes_the_tile():
