@@ -191,21 +191,23 @@ struct StepConfig {
   uint32_t* ufeat;         // [key_cap]
   // Plan regions: region r covers chunks [r*cpr, (r+1)*cpr) of 64 sorted entries (cpr =
   // ceil(chunks / n_regions), from the step's key count); k_seg_plan wave w owns the
-  // n_regions / (unique_grid * NW) regions from w * that count and writes, without
+  // n_regions / (waves of its grid) regions from w * that count and writes, without
   // atomics, each region's short rows (<= kSegShort entries) at srec[r*cpr*64 ...] with
   // count scount[r], one record {first entry, row id, run-start mask (bit i: entry i
   // starts a (row, batch) run), len | batch of run j << (6 + 3j)}, and its medium rows
   // (more entries, inside the 128-entry window, at most 2 per chunk) at mrec[r*cpr*2 ...]
-  // with count mcount[r], {first entry, len}.  k_seg_update's wave w takes region w and,
-  // when there are more regions than waves, further ones from the StepState queue
-  // reg_next, so its blocks need not all be resident at once.
+  // with count mcount[r], {first entry, len}.  Regions, or parts of them, are dealt to the
+  // waves of the row kernels; k_seg_update's wave w takes region w and, when there are more
+  // regions than waves, further ones from the StepState queue reg_next, so its blocks need
+  // not all be resident at once.
   uint4* srec;             // [srec_cap]
   uint32_t srec_cap;
   uint2* mrec;             // [mrec_cap]
   uint32_t mrec_cap;
   uint32_t* scount;        // [n_regions]
   uint32_t* mcount;        // [n_regions]
-  uint32_t n_regions;      // a multiple of unique_grid * NW
+  uint32_t n_regions;      // a multiple of unique_grid * NW (fewer, one per wave of the plan's
+                           // grid, where the step's capacity has fewer chunks of 64 keys)
   // Long rows (running past the window, so at least 65 entries): first sorted entry,
   // first piece, run count and per run (piece count | batch << 24) and its entry count.
   // Only runs of more than kPieceEntries entries are cut into pieces (a piece is a range

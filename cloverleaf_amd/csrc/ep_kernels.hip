@@ -1034,7 +1034,9 @@ __device__ inline void forward_other_loss(const StepConfig& c, StepState* st, ui
 // count) instead of reading k_scan's: up to kForwardOffsets anchors, whose counts a block reads
 // in a few coalesced loads at its start, long before it needs the sum.  The mean model with
 // neighbour rows at fixed places; attention's block map needs the scans.  MI355X, 128 anchors:
-// k_scan took 9.4 us of a 120 us step; at 8192 anchors the blocks would read 270 MB.
+// k_scan took 9.4 us of a 120 us step; a step of 2048 anchors of 8 features at most takes 90 us
+// with D = 8 (96 with k_scan), 91 with D = 64 (96), 97 with D = 128 (103), of 32 features 303
+// (308); at 8192 anchors the blocks would read 270 MB.
 constexpr uint32_t kForwardOffsets = 2048;
 __host__ __device__ inline bool forward_offsets(const StepConfig& c) {
   return c.model == 0 && c.batch <= kForwardOffsets && !(c.nbr_rows && (c.all_nbrs || c.pnbrs));
@@ -2355,7 +2357,8 @@ __device__ inline void count_rows(unsigned long long* slots, uint32_t x) {
 // NZ: the gradient-noise path (noise > 0), built for one tile per width only: its
 // Philox and transcendental code would raise every tile's VGPRs (and cut its waves).
 // blk of grid blocks run the short rows (the whole grid of k_seg_update, part of k_rows').
-template <int D, int VPL, int U, bool H, bool NZ>
+// Q: more regions than waves go through the queue.
+template <int D, int VPL, int U, bool H, bool NZ, bool Q>
 __device__ inline void short_rows(const StepConfig& c, StepState* st, const uint32_t* __restrict__ Ss, uint32_t blk,
                                   uint32_t grid) {
   static_assert(D % VPL == 0 && VPL % 4 == 0 && D / VPL <= 64, "float4 lane slices");
@@ -2382,13 +2385,15 @@ __device__ inline void short_rows(const StepConfig& c, StepState* st, const uint
   __syncthreads();
   const bool noisy = c.noise > 1e-9f;
   uint32_t done = 0;
-  // More regions than waves: wave gw takes region gw, then regions waves, waves + 1, ... from
-  // the queue.  Otherwise a region's rows are dealt to `split` units (unit u takes the row
-  // groups sub, sub + split, ... of region u % nreg, sub = u / nreg) and wave gw takes units
-  // gw, gw + waves, ...: no atomics, and no wave holds the up to 64 rows that start in one
-  // chunk of cold keys while others hold none.
+  // k_seg_update's steps of 8 regions per wave: wave gw takes region gw, then regions waves,
+  // waves + 1, ... from the queue.  Otherwise a region's rows are dealt to `split` units (unit u
+  // takes the row groups sub, sub + split, ... of region u % nreg, sub = u / nreg) and wave gw
+  // takes units gw, gw + waves, ...: no atomics, and no wave holds the up to 64 rows that start
+  // in one chunk of cold keys while others hold none.  k_rows' steps have fewer than 7 regions
+  // per wave, and all of its waves would be at the queue at the same time: 0.47M keys of D = 64
+  // 134 us through it, 38 dealt out.
   const uint32_t nwv = grid * NW;
-  const bool queued = nreg > nwv;
+  const bool queued = Q && nreg > nwv;
   uint32_t split = 1u;
   if (!queued)
     while (split < kUpdSplitMax && nreg * split < kUpdUnitsPerWave * nwv) split *= 2u;
@@ -2611,7 +2616,7 @@ __device__ inline void short_rows(const StepConfig& c, StepState* st, const uint
 
 template <int D, int VPL, int U, bool H, bool NZ = false>
 __global__ __launch_bounds__(256) void k_seg_update(StepConfig c, StepState* st, const uint32_t* __restrict__ Ss) {
-  short_rows<D, VPL, U, H, NZ>(c, st, Ss, blockIdx.x, gridDim.x);
+  short_rows<D, VPL, U, H, NZ, true>(c, st, Ss, blockIdx.x, gridDim.x);
 }
 
 // Loads row f's optimizer operands (whole-wave slice layout).
@@ -2889,7 +2894,7 @@ __global__ __launch_bounds__(256) void k_rows(StepConfig c, StepState* st, const
   const uint32_t b = blockIdx.x;
   if (b < nmed) medium_rows<D, H>(c, st, Ks, Ss, b, nmed);
   else if (b < nmed + npiece) piece_sums<D, H>(c, st, Ss, b - nmed, npiece);
-  else short_rows<D, kRowsVpl, kRowsUnroll, H, false>(c, st, Ss, b - nmed - npiece, gridDim.x - nmed - npiece);
+  else short_rows<D, kRowsVpl, kRowsUnroll, H, false, false>(c, st, Ss, b - nmed - npiece, gridDim.x - nmed - npiece);
 }
 
 // One wave per long row: loads theta/m/v once, adds the pieces of each run in order and
@@ -3427,8 +3432,11 @@ bool seg_variant_supported(int d, int vpl, int unroll) {
 // Steps of few enough keys for one launch of the row kernels (k_rows); a tile asked for by
 // name, the tuner's candidates and gradient noise have k_seg_update instances of their own.
 // MI355X, one launch against two: 16k keys of D = 64 11.8 against 21.2 us, 0.4M keys of
-// D = 128 45 against 60; at D = 768 (256 VGPRs, one wave per SIMD for every role) it gains
-// nothing, so the attention widths past 256 keep two.
+// D = 128 45 against 60; whole steps near 2M keys at capacity (0.67M to 0.84M in the step):
+// D = 8 162 against 175 us and 231 against 245, D = 64 163 / 168 and 224 / 240, D = 128 183 / 197
+// and 245 / 271, D = 256 246 / 258 and 343 / 363, 2048 anchors' hot rows of D = 64 136 / 145.
+// Larger steps were not measured in one.  At D = 768 (256 VGPRs, one wave per SIMD for every
+// role) it gains nothing, so the attention widths past 256 keep two.
 bool rows_in_one_launch(const StepConfig& c) {
   return c.any_tile && c.dims <= 256 && c.key_cap <= kRowsOneLaunch && !(c.noise > 1e-9f);
 }

@@ -61,8 +61,8 @@ def test_one_launch_equals_separate_kernels(dims, form, concurrent):
 
 @pytest.mark.parametrize("dims,form", [(64, "fp32"), (64, "master-fp16"), (256, "fp32"), (256, "bf16")])
 def test_more_regions_than_waves(dims, form):
-    """Enough 64-key regions that the one launch's waves take them from a queue: between 5120
-    (its short-row waves) and 8192 regions."""
+    """Several regions for some of the one launch's waves: between 5120 (its short-row waves)
+    and 8192 regions of 64 keys."""
     prob = make_problem(seed=dims + 1, n=3000, V=30_000, D=dims, fmax=16, zipf=0.7)
     anchors = np.random.default_rng(3).integers(0, prob.n, size=4800).astype(np.uint32)
     samples, one = run(prob, form, 1, (0, 0), anchors, None)
@@ -73,3 +73,24 @@ def test_more_regions_than_waves(dims, form):
     assert 5200 * 64 < keys < 8192 * 64 and np.count_nonzero(one[0]) > 4700
     for a, b in zip(one, separate):
         assert np.array_equal(a, b)
+
+
+def test_one_launch_is_no_slower_with_more_regions_than_waves():
+    """0.45M keys: the row kernels' time of one launch against that of the separate ones.  With
+    the regions past its waves taken from a queue its short rows took 134 us where they take 38 now."""
+    prob = make_problem(seed=8, n=4800, V=3000, D=64, fmax=16, zipf=0.9)
+    ms = []
+    for tile in ((0, 0), (4, 8)):
+        cfg = N.default_config()
+        cfg.dims, cfg.batch_size, cfg.negatives, cfg.gamma, cfg.valid_pct = 64, 4800, K, 3.0, 0.0
+        cfg.alpha = 1e-3  # the examples stay active
+        cfg.max_nodes_kind, cfg.max_nodes, cfg.grad_mode = N.EP_SAMPLE_FIXED, S, N.EP_GRAD_EXACT
+        cfg.seg_vpl, cfg.seg_unroll = tile
+        with N.Context(cfg) as ctx:
+            ctx.set_graph(prob.indptr, prob.indices)
+            ctx.set_features(prob.f_indptr, prob.f_ids, prob.V)
+            ctx.set_table(prob.table)
+            runs = [ctx.bench_steps(2, 10, instrument=True) for _ in range(5)]
+        ms.append(np.median([sum(r.ms_phase[5:8]) for r in runs]))
+    print(f"one launch {ms[0]:.4f} ms, separate {ms[1]:.4f}", flush=True)
+    assert ms[0] < 1.25 * ms[1]
