@@ -498,6 +498,7 @@ int place_step_buffers(ep_ctx* c, uint32_t batch, ep::StepConfig& b, Place&& pla
     if (nrows) EP_TRY(place(&b.nbr_selw, std::max<uint64_t>(c->n_entries, 1)));
   }
   b.nrow_base = batch * NC;
+  b.nrow_cap = (uint32_t)nrow_cap;
   if (att) {
     const uint32_t dm = cfg.dims;
     EP_TRY(place(&b.blkoff, batch + 1));

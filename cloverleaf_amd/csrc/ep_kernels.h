@@ -116,6 +116,7 @@ struct StepConfig {
   int wavg;                // weighted_neighbor_averaging
   int wsample;             // weighted_neighbor_sampling
   uint32_t nrow_base;      // first per-neighbour adjoint row
+  uint32_t nrow_cap;       // per-neighbour adjoint rows there is room for
   // max_features (utils.rs:193-216, model.rs:264-269): 0 All, 1 Fixed(mf_k), 2
   // Probability(mf_p); every node of an example keeps a subset of its (at most 64)
   // features, each kept occurrence counting weight + scale

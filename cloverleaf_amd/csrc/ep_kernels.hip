@@ -756,6 +756,8 @@ __global__ __launch_bounds__(1024) void k_scan(StepConfig c, StepState* st) {
       c.blkoff[c.batch] = s_carry2 <= c.blk_cap ? s_carry2 : 0u;
       if (s_carry2 > c.blk_cap) { st->err = 1u; st->n_keys = c.key_cap + 1u; }
     }
+    // neighbour rows past the capacity: none is written (k_forward)
+    if (nrows && s_carry3 > c.nrow_cap) { st->err = 1u; st->n_keys = c.key_cap + 1u; }
   }
 }
 
@@ -1475,7 +1477,7 @@ __global__ __launch_bounds__(256) void k_forward(StepConfig c, StepState* st) {
     }
   }
   }
-  if (c.nbr_rows) {
+  if (c.nbr_rows && nkeys <= c.key_cap) {  // own_off's rows always fit (nkeys is 0 here)
     // neighbour j's adjoint row is (dL/dp / sum of counts) * (w_j + s_j)
     __syncthreads();
     if (s_el[1]) {
@@ -1704,19 +1706,25 @@ __device__ inline uint64_t digit_peers(bool act, uint32_t d) {
   return act ? peers : 0ull;
 }
 
-// Pass 0 reads the emitted keys (st->n_keys, sentinels included) and drops the sentinels;
-// later passes read the st->n_real compacted keys.
+// Pass 0 reads the emitted keys (st->n_keys, sentinels included; none were emitted where they
+// exceed the capacity) and drops the sentinels; later passes read the st->n_real compacted keys.
+__device__ inline uint32_t sort_count(const StepState* st, int pass, uint32_t key_cap) {
+  if (pass) return st->n_real;
+  return st->n_keys <= key_cap ? st->n_keys : 0u;
+}
+
 // Besides its own counts a block adds them to its group's totals.  Totals of the whole grid
 // took one table: at 20 ns per block and line of it (blocks of all XCDs), 31 us of a pass at
 // 1536 blocks.
 template <int RB>
-__global__ __launch_bounds__(256) void k_rs_hist(const uint32_t* __restrict__ kin, StepState* st, uint32_t* ghist, uint32_t* dgrp,
-                                                 int pass, int shift, int G, uint32_t sent) {
+__global__ __launch_bounds__(256) void k_rs_hist(const uint32_t* __restrict__ kin, StepState* st, uint32_t* ghist,
+                                                 uint32_t* dgrp, int pass, int shift, int G, uint32_t sent,
+                                                 uint32_t key_cap) {
   constexpr uint32_t BINS = 1u << RB, MASK = BINS - 1u;
   __shared__ uint32_t h[BINS];
   const int tid = threadIdx.x, lane = tid & 63;
   uint32_t lo, hi;
-  block_range(pass == 0 ? st->n_keys : st->n_real, G, blockIdx.x, &lo, &hi);
+  block_range(sort_count(st, pass, key_cap), G, blockIdx.x, &lo, &hi);
   if (lo >= hi) return;  // k_rs_scatter reads the counts of blocks with elements only
   for (uint32_t d = tid; d < BINS; d += 256u) h[d] = 0u;
   __syncthreads();
@@ -1773,7 +1781,7 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const uint32_t* __restrict__
                                                     uint32_t* __restrict__ kout, uint32_t* __restrict__ vout,
                                                     StepState* st, const uint32_t* __restrict__ ghist,
                                                     const uint32_t* __restrict__ dgrp, int pass,
-                                                    int shift, int G, uint32_t sent) {
+                                                    int shift, int G, uint32_t sent, uint32_t key_cap) {
   constexpr uint32_t BINS = 1u << RB, MASK = BINS - 1u;
   constexpr int IT = RS_SCATTER_ITEMS;
   constexpr uint32_t TILE = 256u * IT;
@@ -1785,7 +1793,7 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const uint32_t* __restrict__
   __shared__ uint32_t lk[TILE], lv[TILE];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   uint32_t lo, hi;
-  block_range(pass == 0 ? st->n_keys : st->n_real, G, blockIdx.x, &lo, &hi);
+  block_range(sort_count(st, pass, key_cap), G, blockIdx.x, &lo, &hi);
   if (lo >= hi) return;
   {
     // thread tid owns digits [tid * DPT, tid * DPT + DPT)
@@ -3380,9 +3388,9 @@ static void launch_sort_rb(const StepConfig& c, StepState* st, hipStream_t s, in
   for (int p = 0; p < passes; ++p) {
     const int shift = p * RB;
     hipLaunchKernelGGL((k_rs_hist<RB>), dim3(G), dim3(256), 0, s, c.keys[*cur], st, c.ghist, c.dgrp, p, shift, G,
-                       c.sentinel);
+                       c.sentinel, c.key_cap);
     hipLaunchKernelGGL((k_rs_scatter<RB>), dim3(G), dim3(256), 0, s, c.keys[*cur], c.slots[*cur], c.keys[1 - *cur],
-                       c.slots[1 - *cur], st, c.ghist, c.dgrp, p, shift, G, c.sentinel);
+                       c.slots[1 - *cur], st, c.ghist, c.dgrp, p, shift, G, c.sentinel, c.key_cap);
     *cur = 1 - *cur;
   }
 }
