@@ -347,7 +347,10 @@ struct ep_ctx {
     void* q = nullptr;
     const size_t bytes = std::max<size_t>(count * sizeof(T), 16);
     hipError_t e = hipMalloc(&q, bytes);
-    if (e != hipSuccess) return fail(EP_ENOMEM, "hipMalloc(" + std::to_string(bytes) + " bytes) failed: " + hipGetErrorString(e));
+    if (e != hipSuccess) {
+      (void)hipGetLastError();  // not the next launch's error
+      return fail(EP_ENOMEM, "hipMalloc(" + std::to_string(bytes) + " bytes) failed: " + hipGetErrorString(e));
+    }
     allocs.push_back(q);
     *p = (T*)q;
     return EP_OK;
@@ -612,7 +615,8 @@ int ensure_step_buffers(ep_ctx* c, uint32_t batch) {
   if (!c->d_indptr || !c->d_findptr) return fail(EP_ESTATE, "graph and features must be set first");
   const ep_config& cfg = c->cfg;
   const uint32_t D = row_width(cfg);
-  // drop old buffers
+  // drop old buffers; a later call places them again also where this one runs out of memory
+  c->cap_batch = 0;
   ep::StepConfig& b = c->base;
   c->release(b.nbr_cnt); c->release(b.nbr); c->release(b.neg); c->release(b.rcount); c->release(b.keyoff);
   c->release(b.ex_fs); c->release(b.ex_fn);
@@ -638,7 +642,8 @@ int ensure_step_buffers(ep_ctx* c, uint32_t batch) {
   // (row, batch) run); they are allocated by ep_step_explicit on first use
   c->unique_cap = std::min<uint64_t>((uint64_t)c->n_vocab * P, keycap) + 1;
   EP_TRY(c->alloc(&c->d_explicit, batch));
-  if (!b.Gd && cfg.scatter == EP_SCATTER_ATOMIC) {
+  if (!b.touched && cfg.scatter == EP_SCATTER_ATOMIC) {
+    c->release(b.Gd); c->release(b.flag);
     EP_TRY(c->alloc(&b.Gd, (size_t)c->n_vocab * D));
     EP_TRY(c->alloc(&b.flag, c->n_vocab));
     EP_TRY(c->alloc(&b.touched, c->n_vocab));
