@@ -669,9 +669,10 @@ __device__ inline void att_random_setup(const StepConfig& c, const StepState* st
 // ------------------------------------------------------------------------------------
 // k_att_forward: one wave (64-thread block) per attention block.  Four waves per SIMD asked
 // for: the compiler then keeps the matrix results out of accumulation registers (122 VGPRs
-// in all, no spills; 143 without; Sliding and Random would spill and are left to it).  31.7k blocks of 32 items on average, 4 heads, d_k 32, d 128, FP32:
-// 560 -> 348 us with one matrix product per tile pair instead of two (see put_tile); what is
-// left is the latency of the row loads and the softmax of the padded tiles.
+// in all, no spills; 143 without; Sliding and Random would spill and are left to it).  31.7k
+// blocks of 32 items on average, 4 heads, d_k 32, d 128, FP32: 560 -> 348 us with one matrix
+// product per tile pair instead of two (see put_tile); what is left is the latency of the row
+// loads and the softmax of the padded tiles.
 // ------------------------------------------------------------------------------------
 template <int DK, typename T, int AM>
 __global__ __launch_bounds__(64, AM == AM_FULL ? 4 : 1) void k_att_forward(StepConfig c, StepState* st) {
@@ -693,10 +694,12 @@ __global__ __launch_bounds__(64, AM == AM_FULL ? 4 : 1) void k_att_forward(StepC
 // without the bound): 40k nodes of 16 features, 446 -> 277 us with k_att_forward's change.
 // ------------------------------------------------------------------------------------
 template <int DK, typename T, int AM>
-__global__ __launch_bounds__(64, AM == AM_FULL ? 3 : 1) void k_att_embed(const T* __restrict__ table, uint32_t W, int H, int dm,
-                                                  const uint64_t* __restrict__ findptr,
-                                                  const uint32_t* __restrict__ fids, uint64_t n_nodes,
-                                                  uint32_t win, float* __restrict__ out) {
+__global__ __launch_bounds__(64, AM == AM_FULL ? 3 : 1) void k_att_embed(const T* __restrict__ table, uint32_t W,
+                                                                        int H, int dm,
+                                                                        const uint64_t* __restrict__ findptr,
+                                                                        const uint32_t* __restrict__ fids,
+                                                                        uint64_t n_nodes, uint32_t win,
+                                                                        float* __restrict__ out) {
   extern __shared__ float sm[];
   const AttLds L = att_lds(sm, dm, H, win, false);
   const uint32_t lane = lane_id();

@@ -580,7 +580,8 @@ int place_step_buffers(ep_ctx* c, uint32_t batch, ep::StepConfig& b, Place&& pla
     b.fuse_hash = fh;
     b.fuse_max = fh / 8 * 5;
     const uint64_t entries = 1ull + neighbour_cap(c) + K;
-    b.fuse_all = !att && entries <= ent_cap && rmax <= b.ids_cap && (cfg.grad_mode != EP_GRAD_FIRST_LEAF || rmax <= b.fuse_max);
+    b.fuse_all = !att && entries <= ent_cap && rmax <= b.ids_cap &&
+                 (cfg.grad_mode != EP_GRAD_FIRST_LEAF || rmax <= b.fuse_max);
   }
   b.unique_grid = unique_grid;
   *keycap_out = keycap;
@@ -624,7 +625,8 @@ int ensure_step_buffers(ep_ctx* c, uint32_t batch) {
   c->release(b.adj); c->release(b.adjh); c->release(b.ascale); c->release(b.coef); c->release(b.elig);
   c->release(b.loss);
   c->release(b.keys[0]); c->release(b.keys[1]); c->release(b.slots[0]); c->release(b.slots[1]);
-  c->release(b.ghist); c->release(b.dgrp); c->release(b.G); c->release(b.ufeat); c->release(b.long_st); c->release(b.long_len);
+  c->release(b.ghist); c->release(b.dgrp); c->release(b.G); c->release(b.ufeat);
+  c->release(b.long_st); c->release(b.long_len);
   c->release(b.long_pbase); c->release(b.long_runs); c->release(b.long_rlen); c->release(b.piece_st);
   c->release(b.piece_info);
   c->release(b.part); c->release(b.srec); c->release(b.mrec); c->release(b.scount); c->release(b.mcount);
@@ -1702,7 +1704,8 @@ struct RunCounts : ep::StepHead {
 static int read_counts(ep_ctx* c, RunCounts* out) {
   std::vector<unsigned long long> upd(std::size(c->d_state->upd_short) + std::size(c->d_state->upd_long));
   EP_HIP(hipMemcpy((ep::StepHead*)out, c->d_state, sizeof(ep::StepHead), hipMemcpyDeviceToHost));
-  static_assert(sizeof(ep::StepState::upd_short) == sizeof(ep::StepState::upd_long), "two counter tables, one after the other");
+  static_assert(sizeof(ep::StepState::upd_short) == sizeof(ep::StepState::upd_long),
+                "two counter tables, one after the other");
   EP_HIP(hipMemcpy(upd.data(), c->d_state->upd_short, upd.size() * sizeof(upd[0]), hipMemcpyDeviceToHost));
   out->rows = out->stat_unique;
   out->short_rows = 0;
@@ -1866,7 +1869,8 @@ int ep_embed_weighted(ep_ctx* c, uint64_t n_nodes, const uint64_t* f_indptr, con
   if (!(alpha > 0.f) || !std::isfinite(alpha)) return fail(EP_EINVAL, "alpha must be finite and > 0");
   for (uint64_t i = 0; i < n_nodes; ++i)
     if (f_indptr[i + 1] < f_indptr[i]) return fail(EP_EINVAL, "f_indptr must be non-decreasing");
-  if (!ids_below(f_ids, f_indptr[n_nodes], std::min(c->n_vocab, n_p))) return fail(EP_EINVAL, "feature id out of range");
+  if (!ids_below(f_ids, f_indptr[n_nodes], std::min(c->n_vocab, n_p)))
+    return fail(EP_EINVAL, "feature id out of range");
   for (uint32_t i = 0; i < n_p; ++i)
     if (!(p_w[i] >= 0.f)) return fail(EP_EINVAL, "unigram probabilities must be >= 0");
   return embed_lists(c, n_nodes, f_indptr, f_ids, p_w, n_p, row_width(c->cfg), out,

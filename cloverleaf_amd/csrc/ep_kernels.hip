@@ -3114,7 +3114,8 @@ __global__ __launch_bounds__(256) void k_pack_rows(const float4* __restrict__ sr
 }
 
 // dst[i] = FP32 of the BF16 value src[i], four values per thread (exact), n4 groups of four.
-__global__ __launch_bounds__(256) void k_widen_bf16(const uint2* __restrict__ src, float4* __restrict__ dst, uint64_t n4) {
+__global__ __launch_bounds__(256) void k_widen_bf16(const uint2* __restrict__ src, float4* __restrict__ dst,
+                                                    uint64_t n4) {
   const uint64_t step = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += step) {
     const uint2 t = src[i];
@@ -3312,8 +3313,8 @@ hipError_t launch_sample(const StepConfig& c0, StepState* st, float lr, hipStrea
   int passes, rb;
   radix_plan(c.sort_bits, &passes, &rb);
   c.sort_totals = c.train ? ((uint32_t)passes * sort_groups(c.sort_grid)) << rb : 0u;
-  hipLaunchKernelGGL(k_sample, dim3((c.batch + NW - 1) / NW + 1), dim3(256), (size_t)NW * c.S * sizeof(uint32_t), s, c, st,
-                     lr);
+  hipLaunchKernelGGL(k_sample, dim3((c.batch + NW - 1) / NW + 1), dim3(256), (size_t)NW * c.S * sizeof(uint32_t), s, c,
+                     st, lr);
   return hipGetLastError();
 }
 
@@ -3494,8 +3495,9 @@ static void launch_row_kernels(const StepConfig& c, StepState* st, int buf, hipS
     const uint32_t nmed = (uint32_t)std::min(wave_grid(1), c.unique_grid / 8);
     const uint32_t npiece = (uint32_t)std::min(wave_grid(2), c.unique_grid / 4);
     const uint32_t nshort = (uint32_t)std::min<uint64_t>(wave_grid(kUpdSplitMax), c.unique_grid - nmed - npiece);
-    if constexpr (D <= 256) hipLaunchKernelGGL((k_rows<D, H>), dim3(nmed + npiece + nshort), dim3(256), 0, s, c, st, c.keys[buf], c.slots[buf],
-                       npiece, nmed);
+    if constexpr (D <= 256)
+      hipLaunchKernelGGL((k_rows<D, H>), dim3(nmed + npiece + nshort), dim3(256), 0, s, c, st, c.keys[buf],
+                         c.slots[buf], npiece, nmed);
     if (ev) (void)hipEventRecord(ev[1], s);
     if (ev) (void)hipEventRecord(ev[2], s);
     hipLaunchKernelGGL((k_long_combine<D, H>), dim3(lgrid), dim3(256), 0, s, c, st, c.keys[buf], c.slots[buf]);
