@@ -74,6 +74,8 @@ __device__ inline void store_adj_row(const StepConfig& c, size_t slot, int lane,
   }
 }
 
+__device__ inline uint32_t wave_uniform(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
+
 // First index i in [lo, hi) with K[i] >= x (hi if none), K sorted; 64-ary search by
 // the whole wave.
 __device__ inline uint32_t wave_lower_bound(const uint32_t* __restrict__ K, uint32_t lo, uint32_t hi, uint32_t x) {
@@ -2343,19 +2345,21 @@ __global__ __launch_bounds__(256) void k_seg_plan(StepConfig c, StepState* st, c
 }
 
 // Adds the block's rows updated (x summed over its threads) to its own counter slot: blocks
-// of one stream's kernels follow each other, so no atomics.  One 64-bit atomic per wave on
-// one address serialised thousands of waves at the end of every row kernel.
-__device__ inline void count_rows(unsigned long long* slots, uint32_t x) {
-  __shared__ uint32_t s_cnt[NW];
+// of one stream's kernels follow each other, so no global atomics (one 64-bit atomic per wave
+// on one address serialised thousands of waves at the end of every row kernel).  The waves add
+// up in LDS, the last one to arrive writes: a barrier would hold the registers of the block's
+// finished waves until its slowest (the 50M-node workload's short rows 1% longer).  cnt is 0
+// before the block's last barrier (clear_count).
+__device__ inline void clear_count(unsigned long long* cnt) {
+  if (threadIdx.x == 0u) *cnt = 0ull;
+}
+__device__ inline void count_rows(unsigned long long* cnt, unsigned long long* slots, uint32_t x) {
+  constexpr uint32_t kWaves = 48;  // bits of the rows; the waves that have arrived above them
   x = wave_sum_u32(x);
-  if ((threadIdx.x & 63u) == 0u) s_cnt[threadIdx.x >> 6] = x;
-  __syncthreads();
-  if (threadIdx.x == 0u) {
-    uint32_t t = 0u;
-#pragma unroll
-    for (int q = 0; q < NW; ++q) t += s_cnt[q];
-    if (t) slots[blockIdx.x] += t;
-  }
+  if ((threadIdx.x & 63u) != 0u) return;
+  const unsigned long long was = atomicAdd(cnt, (1ull << kWaves) | x);
+  const unsigned long long t = (was & ((1ull << kWaves) - 1ull)) + x;
+  if ((was >> kWaves) == (unsigned long long)(NW - 1) && t) slots[blockIdx.x] += t;
 }
 
 // Short rows: lane groups of L = D/VPL lanes (VPL values per lane as VPL/4 float4
@@ -2375,6 +2379,8 @@ __device__ inline void short_rows(const StepConfig& c, StepState* st, const uint
   constexpr int NQ = VPL / 4;     // float4 columns per lane
   constexpr int NS = ((int)kSegShort + L - 1) / L;  // slots held per lane
   __shared__ float s_lr[kMaxGroup];
+  __shared__ unsigned long long s_cnt;
+  clear_count(&s_cnt);
   const int tid = threadIdx.x, lane = tid & 63;
   const int grp = lane / L, lg = lane % L;
   const bool gact = grp < G;
@@ -2407,11 +2413,12 @@ __device__ inline void short_rows(const StepConfig& c, StepState* st, const uint
     while (split < kUpdSplitMax && nreg * split < kUpdUnitsPerWave * nwv) split *= 2u;
   const uint32_t units = nreg * split;
   const uint32_t stride = (uint32_t)G * split;  // rows between two of a lane group's
-  for (uint32_t unit = blk * NW + (uint32_t)(tid >> 6);;) {
+  // (unit, and what follows from it, in scalar registers)
+  for (uint32_t unit = wave_uniform(blk * NW + (uint32_t)(tid >> 6));;) {
     if (unit >= units) break;
     const uint32_t reg = queued ? unit : unit % nreg;
     const uint32_t first = queued ? 0u : unit / nreg * (uint32_t)G;  // the unit's first row group
-    const uint32_t nrec = c.scount[reg];
+    const uint32_t nrec = wave_uniform(c.scount[reg]);
     const uint4* recs = c.srec + (size_t)reg * cpr * 64u;
     // Software pipeline over the region's rows: iteration k issues, back to back, the row's
     // theta/m/v, the next row's slots (its record arrived one iteration earlier), the
@@ -2617,9 +2624,9 @@ __device__ inline void short_rows(const StepConfig& c, StepState* st, const uint
     }
     uint32_t nx = 0u;
     if (lane == 0) nx = atomicAdd(&st->reg_next, 1u);
-    unit = nwv + (uint32_t)__shfl((int)nx, 0, EP_WAVE);
+    unit = nwv + wave_uniform(nx);
   }
-  count_rows(st->upd_short, done);
+  count_rows(&s_cnt, st->upd_short, done);
 }
 
 template <int D, int VPL, int U, bool H, bool NZ = false>
@@ -2709,7 +2716,6 @@ __device__ inline void add_rows_tree(float (&acc)[PL], float (&r)[U][PL], uint32
   for (int q = 0; q < PL; ++q) acc[q] += r[0][q];
 }
 
-__device__ inline uint32_t wave_uniform(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
 __device__ inline uint32_t lane_value(uint32_t x, uint32_t lane) {
   return (uint32_t)__builtin_amdgcn_readlane((int)x, (int)lane);
 }
@@ -2816,6 +2822,8 @@ __device__ inline void medium_rows(const StepConfig& c, StepState* st, const uin
   constexpr int PL = RowShape<D>::PL;
   constexpr int U = SR_UNROLL;
   __shared__ float s_lr[kMaxGroup], s_sd[kMaxGroup];
+  __shared__ unsigned long long s_cnt;
+  clear_count(&s_cnt);
   const int lane = threadIdx.x & 63;
   const uint32_t gw = blk * NW + wave_uniform(threadIdx.x >> 6);
   const uint32_t nwaves = grid * NW;
@@ -2883,7 +2891,7 @@ __device__ inline void medium_rows(const StepConfig& c, StepState* st, const uin
       }
     }
   }
-  count_rows(st->upd_long, lane == 0 ? done : 0u);
+  count_rows(&s_cnt, st->upd_long, lane == 0 ? done : 0u);
 }
 
 template <int D, bool H>
@@ -2920,6 +2928,8 @@ __global__ __launch_bounds__(256) void k_long_combine(StepConfig c, StepState* s
   const uint32_t nl = st->n_long < c.long_cap ? st->n_long : c.long_cap;
   const StepScalars sv = step_scalars(st);
   __shared__ float s_lr[kMaxGroup], s_sd[kMaxGroup];
+  __shared__ unsigned long long s_cnt;
+  clear_count(&s_cnt);
   if (threadIdx.x < kMaxGroup) {
     s_lr[threadIdx.x] = st->lr[threadIdx.x];
     s_sd[threadIdx.x] = st->noise_sd[threadIdx.x];
@@ -2969,7 +2979,7 @@ __global__ __launch_bounds__(256) void k_long_combine(StepConfig c, StepState* s
       ++done;
     }
   }
-  count_rows(st->upd_long, lane == 0 ? done : 0u);
+  count_rows(&s_cnt, st->upd_long, lane == 0 ? done : 0u);
 }
 
 // ------------------------------------------------------------------------------------
