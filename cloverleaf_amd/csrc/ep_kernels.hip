@@ -2504,7 +2504,9 @@ __device__ inline void short_rows(const StepConfig& c, StepState* st, const uint
         for (uint32_t u0 = 0; u0 < maxlen; u0 += U) {
           // entries past the run skip their loads (a wave-uniform branch when G == 1: most
           // runs of short rows are 1-3 entries long, whose loads all issue before a wait)
-          float4 r[U][NQ];
+          float4 r[H ? 1 : U][NQ];
+          uint2 t16[H ? U : 1][NQ];  // FP16 rows stay as loaded until they are added
+          float sc[H ? U : 1];
   #pragma unroll
           for (int u = 0; u < U; ++u) {
             const uint32_t e = a + u0 + (uint32_t)u;
@@ -2521,13 +2523,11 @@ __device__ inline void short_rows(const StepConfig& c, StepState* st, const uint
             }
             slot &= kSlotMask;
             if constexpr (H) {
-              const float sc = valid ? c.ascale[slot] : 0.f;
+              sc[u] = valid ? c.ascale[slot] : 0.f;
   #pragma unroll
               for (int q = 0; q < NQ; ++q) {
                 const uint32_t col = (uint32_t)(q * L + lg) * 4u;
-                const uint2 t = valid ? *reinterpret_cast<const uint2*>(c.adjh + (size_t)slot * D + col) : make_uint2(0u, 0u);
-                r[u][q] = make_float4(sc * f16_to_f32((uint16_t)(t.x & 0xffffu)), sc * f16_to_f32((uint16_t)(t.x >> 16)),
-                                      sc * f16_to_f32((uint16_t)(t.y & 0xffffu)), sc * f16_to_f32((uint16_t)(t.y >> 16)));
+                t16[u][q] = valid ? *reinterpret_cast<const uint2*>(c.adjh + (size_t)slot * D + col) : make_uint2(0u, 0u);
               }
             } else {
   #pragma unroll
@@ -2542,7 +2542,18 @@ __device__ inline void short_rows(const StepConfig& c, StepState* st, const uint
           for (int u = 0; u < U; ++u) {
   #pragma unroll
             for (int q = 0; q < NQ; ++q) {
-              acc[q].x += r[u][q].x; acc[q].y += r[u][q].y; acc[q].z += r[u][q].z; acc[q].w += r[u][q].w;
+              float4 x;
+              if constexpr (H) {
+                // a fence as below: widened where it was loaded, a row's load is waited for inside
+                // its branch (tiles of 8 and 16 values: 20 ms against 10.5 at the 50M-node shape)
+                uint32_t tx = t16[u][q].x, ty = t16[u][q].y;
+                asm volatile("" : "+v"(tx), "+v"(ty));
+                x = make_float4(sc[u] * f16_to_f32((uint16_t)(tx & 0xffffu)), sc[u] * f16_to_f32((uint16_t)(tx >> 16)),
+                                sc[u] * f16_to_f32((uint16_t)(ty & 0xffffu)), sc[u] * f16_to_f32((uint16_t)(ty >> 16)));
+              } else {
+                x = r[u][q];
+              }
+              acc[q].x += x.x; acc[q].y += x.y; acc[q].z += x.z; acc[q].w += x.w;
             }
           }
         }
@@ -2738,7 +2749,7 @@ __device__ inline RowNames<H> row_names(const StepConfig& c, uint32_t slot) {
 // a half, its row's scale and the partner's product: the scales are powers of two, so the
 // products are exact and the sum is rounded once, as an add of widened rows is.  At D = 256
 // about 9 vector instructions per row against 30.  Pieces of the 10M-node shape (FP32 rows of
-// 256) 494 -> 410 us, of the 50M-node shape (FP16 rows) 4.94 -> 4.57 ms, there at 6.2 TB/s of
+// 256) 494 -> 410 us, of the 50M-node shape (FP16 rows) 4.94 -> 4.57 ms, there at 7.0 TB/s of
 // rows that miss the L2, which is what bounds them.
 template <int D, bool H, int U>
 __device__ inline void add_named_rows(const StepConfig& c, const RowNames<H>& names, uint32_t t0, uint32_t n, int lane,

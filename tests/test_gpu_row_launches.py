@@ -94,3 +94,24 @@ def test_one_launch_is_no_slower_with_more_regions_than_waves():
         ms.append(np.median([sum(r.ms_phase[5:8]) for r in runs]))
     print(f"one launch {ms[0]:.4f} ms, separate {ms[1]:.4f}", flush=True)
     assert ms[0] < 1.25 * ms[1]
+
+
+def test_wide_fp16_tiles_keep_their_loads_in_flight():
+    """FP16 adjoint rows of 256 with 16 values a lane, short rows alone, against 4 values.  With
+    each row's load waited for inside its own branch they took 2.7 times as long."""
+    prob = make_problem(seed=9, n=3000, V=200_000, D=256, fmax=32, zipf=0.5)
+    ms = []
+    for tile in ((4, 8), (16, 2)):
+        cfg = N.default_config()
+        cfg.precision, cfg.fp16_adjoints = N.EP_PREC_BF16, 1
+        cfg.dims, cfg.batch_size, cfg.negatives, cfg.gamma, cfg.valid_pct = 256, 3000, K, 3.0, 0.0
+        cfg.alpha = 1e-3
+        cfg.max_nodes_kind, cfg.max_nodes, cfg.grad_mode = N.EP_SAMPLE_FIXED, S, N.EP_GRAD_EXACT
+        cfg.seg_vpl, cfg.seg_unroll = tile
+        with N.Context(cfg) as ctx:
+            ctx.set_graph(prob.indptr, prob.indices)
+            ctx.set_features(prob.f_indptr, prob.f_ids, prob.V)
+            ctx.set_table(prob.table)
+            ms.append(np.median([ctx.bench_steps(2, 10, instrument=True).ms_phase[5] for _ in range(5)]))
+    print(f"4 values {ms[0]:.4f} ms, 16 values {ms[1]:.4f}", flush=True)
+    assert ms[1] < 1.8 * ms[0]
